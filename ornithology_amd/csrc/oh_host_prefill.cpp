@@ -105,13 +105,15 @@ int pf_alloc(ornith_hip_session *s, int tc) {
     const size_t nch = (s->kvcap + oh_flash_chunk() - 1) / oh_flash_chunk();
     CHK(salloc(s, &p.X, T * H));
     CHK(q8alloc(s, p.XQ, T * H));
-    CHK(salloc(s, &p.CAT, T * cc + 1)); CHK(salloc(s, &p.CONV, T * cc + 1));
+    const size_t T32 = (T + 31) / 32 * 32;   // the delta scan reads whole 32-token chunks
+    CHK(salloc(s, &p.CAT, T * cc + 1)); CHK(salloc(s, &p.CONV, T32 * cc + 1));
     CHK(salloc(s, &p.Z, T * vd + 1)); CHK(salloc(s, &p.O, T * vd + 1));
     CHK(q8alloc(s, p.OQ, T * vd + 256));
     CHK(salloc(s, &p.A, T * a.nv + 1)); CHK(salloc(s, &p.Bg, T * a.nv + 1));
     CHK(salloc(s, &p.AL, T * a.nv + 1)); CHK(salloc(s, &p.BE, T * a.nv + 1));
-    CHK(salloc(s, &p.QN, T * qd + 1)); CHK(salloc(s, &p.KN, T * qd + 1));
-    CHK(salloc(s, &p.GR, (size_t)oh_delta_grams_floats(tc, a.nk > 0 ? a.nk : 1) + 1));
+    CHK(salloc(s, &p.QN, T32 * qd + 1)); CHK(salloc(s, &p.KN, T32 * qd + 1));
+    const int gr = oh_delta_grams_floats(tc, a.nk > 0 ? a.nk : 1), co = oh_delta_coef_floats(tc, a.nv > 0 ? a.nv : 1);
+    CHK(salloc(s, &p.GR, (size_t)(gr > co ? gr : co) + 1));
     CHK(salloc(s, &p.STAGE, (size_t)(a.conv_k > 1 ? a.conv_k - 1 : 1) * cc + 1));
     CHK(salloc(s, &p.QP, T * 2 * aq + 1)); CHK(salloc(s, &p.KB, T * kvd + 1)); CHK(salloc(s, &p.VB, T * kvd + 1));
     CHK(salloc(s, &p.QR, T * aq + 1)); CHK(salloc(s, &p.AG, T * aq + 1)); CHK(salloc(s, &p.OA, T * aq + 1));

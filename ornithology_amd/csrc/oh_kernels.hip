@@ -164,16 +164,7 @@ hipError_t oh_launch_delta_chunked(int dk, const float *qn, const float *kn, con
         }
         return hipGetLastError();
     }
-    if (dk == 128) {
-        hipLaunchKernelGGL(oh_k_delta_grams<128>, gg, dim3(256), 0, st, qn, kn, T, nk, grams);
-        hipLaunchKernelGGL(oh_k_delta_chunked<128>, dim3(nv * 8), dim3(256), 0, st, qn, kn, conv, al, be, grams, S, out, T, nk, nv, cc, out_scale);
-    } else if (dk == 64) {
-        hipLaunchKernelGGL(oh_k_delta_grams<64>, gg, dim3(256), 0, st, qn, kn, T, nk, grams);
-        hipLaunchKernelGGL(oh_k_delta_chunked<64>, dim3(nv * 4), dim3(256), 0, st, qn, kn, conv, al, be, grams, S, out, T, nk, nv, cc, out_scale);
-    } else {
-        return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return oh_launch_delta_exact(dk, qn, kn, conv, al, be, grams, S, out, T, nk, nv, cc, out_scale, st);
 }
 hipError_t oh_launch_delta_batch(const oh_op_delta *ops, const int32_t *pos, int n, int dk, int K, int nv,
                                  hipStream_t st) {

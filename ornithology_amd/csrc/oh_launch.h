@@ -29,9 +29,17 @@ hipError_t oh_launch_qk_gates_rows(int dk, const float *conv, const float *A, co
 hipError_t oh_launch_delta_scan(int dk, const float *qn, const float *kn, const float *conv, const float *al,
                                 const float *be, float *S, float *out, int T, int nk, int nv, int cc,
                                 float out_scale, hipStream_t st);
-// the reference's chunked delta scan (grams per key head and chunk, then the scan)
+// the reference's chunked delta scan: the chunks' coefficients, then the scan.
+// qn, kn and conv hold whole 32-token chunks (allocated, not necessarily
+// written, past row T)
+int oh_delta_coef_floats(int T, int nv);
+hipError_t oh_launch_delta_exact(int dk, const float *qn, const float *kn, const float *conv, const float *al,
+                                 const float *be, float *coef, float *S, float *out, int T, int nk, int nv, int cc,
+                                 float out_scale, hipStream_t st);
+// grams: scratch of at least oh_delta_coef_floats and oh_delta_grams_floats
+// floats; wy non-null: the matrix-core WY form over that scratch
+// (oh_delta_wy_floats), else oh_launch_delta_exact
 int oh_delta_grams_floats(int T, int nk);
-// wy non-null: the matrix-core WY form over that scratch (oh_delta_wy_floats)
 hipError_t oh_launch_delta_chunked(int dk, const float *qn, const float *kn, const float *conv, const float *al,
                                    const float *be, float *grams, float *wy, float *S, float *out, int T, int nk,
                                    int nv, int cc, float out_scale, hipStream_t st);

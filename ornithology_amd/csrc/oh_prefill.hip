@@ -194,17 +194,8 @@ oh_k_delta_scan(const float *qn, const float *kn, const float *conv, const float
     for (int c = 0; c < DK / 4; c++) stg((float4 *)Sr + c, make_float4(s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]));
 }
 
-// ---- chunked delta scan (the reference's default prompt mode) --------------------
-// ornith_delta_prefill / delta_chunk (src/ornith_attn.c:215-349): the prompt in
-// chunks of kDeltaChunk tokens counted from the start of the evaluation; per
-// chunk, with S_in the incoming state,
-//   p_i = prod_{l<=i} alpha_l, Sk_i = S_in k_i, Sq_i = S_in q_i,
-//   u_i = beta_i v_i - beta_i p_i Sk_i - sum_{j<i} beta_i (p_i/p_j)(k_j.k_i) u_j,
-//   o_i = p_i Sq_i + sum_{j<=i} (p_i/p_j)(k_j.q_i) u_j,
-//   S_out = p_{C-1} S_in + sum_j (p_{C-1}/p_j) u_j k_j^T,
-// where p_i/p_j is accumulated as the running product of alpha_{j+1..i}. Every
-// float is formed in the reference's order, so the result equals its bits
-// (it differs from the token-by-token recurrence in rounding).
+// ---- Gram matrices of the matrix-core chunked delta scan (oh_delta_mfma.hip; the
+// reference-order scan forms its own, oh_kernels_delta.hip) ------------------------
 constexpr int kDeltaChunk = 32;
 
 // the chunk Gram matrices, once per (key head, chunk): kk[i][j] = k_j.k_i and
@@ -246,292 +237,6 @@ oh_k_delta_grams(const float *qn, const float *kn, int T, int nk, float *grams) 
     float *g = grams + ((size_t)ch * nk + kh) * 2 * CH * CH;
 #pragma unroll
     for (int m = 0; m < NP; m++) stg(g + tid + 256 * m, acc[m]);
-}
-
-// A block per 16 rows of one value head's state (256 blocks at C3). Thread
-// (r, g) = (tid % 16, tid / 16) keeps state row r in registers and takes
-// tokens g and g + 16 of each chunk for the S_in projections and the outputs;
-// the first 16 threads run the forward substitution of their rows; for the
-// state update thread (tid / 16, tid % 16) owns DK / 16 columns of one row in
-// LDS (the update is independent per element). Every float is formed in
-// delta_chunk's order.
-template <int DK>
-__global__ void __launch_bounds__(256)
-oh_k_delta_chunked(const float *qn, const float *kn, const float *conv, const float *al, const float *be,
-                   const float *grams, float *S, float *out, int T, int nk, int nv, int cc, float out_scale) {
-    constexpr int CH = kDeltaChunk, RB = 16, KS = DK + 4, XS = DK + 4, CPL = DK / 16;
-    __shared__ __align__(16) float kc[CH][KS], qc[CH][KS];
-    __shared__ __align__(16) float M[CH][CH + 4], W[CH][CH + 4];   // k_j.k_i / k_j.q_i, then the coefficients
-    __shared__ float U[CH][RB + 1], Sq[CH][RB + 1];      // [token][row]
-    __shared__ float alpha[CH], beta[CH], p[CH], wend[CH];
-    __shared__ int mz[CH];                               // row i of M holds a zero (j < i)
-    __shared__ __align__(16) float xs[RB * XS];
-    const int tid = tid_x();
-    // blocks go to the 8 XCDs round-robin (XCD = block % 8); with nv % 8 == 0
-    // the slabs of a head share one XCD and its L2 copy of the head's inputs
-    constexpr int NS = DK / RB;
-    const int vb = (int)blockIdx.x;
-    const int hv = (nv & 7) == 0 ? ((vb >> 3) / NS) * 8 + (vb & 7) : vb / NS;
-    const int slab = (nv & 7) == 0 ? (vb >> 3) % NS : vb % NS, kh = hv % nk;
-    const int qd = nk * DK, vd = nv * DK, r0 = hv * DK + slab * RB;
-    const int r = tid % RB, g = tid / RB;                // projections, outputs, reload
-    const int ur = tid / RB, ucg = tid % RB;             // update: row, column group
-    float *Srow = S + (size_t)r0 * DK;
-    for (int e = tid; e < RB * DK / 4; e += 256) {
-        const int row = e / (DK / 4), c4 = e - row * (DK / 4);
-        *(float4 *)(xs + row * XS + 4 * c4) = ldg((const float4 *)Srow + e);
-    }
-    __syncthreads();
-    float s[DK];
-    auto reload = [&]() {
-#pragma unroll
-        for (int c = 0; c < DK / 4; c++) {
-            const float4 v = *(const float4 *)(xs + r * XS + 4 * c);
-            s[4 * c] = v.x; s[4 * c + 1] = v.y; s[4 * c + 2] = v.z; s[4 * c + 3] = v.w;
-        }
-    };
-    // the next chunk's keys, queries, Gram matrices, values and gates are
-    // requested into registers while the current chunk is computed
-    constexpr int NKQ = CH * DK / 4 / 256, NG = CH * CH / 256, NU = CH * RB / 256;
-    float4 rk[NKQ], rq[NKQ];
-    float rm[NG], rw[NG], ru[NU], ral = 0.0f, rbe = 0.0f;
-    auto fetch = [&](int cs, int chn) {
-        const int Cn = T - cs < CH ? T - cs : CH;
-        if (Cn <= 0) return;
-#pragma unroll
-        for (int m = 0; m < NKQ; m++) {
-            const int e = tid + 256 * m, i = e / (DK / 4), c = e - i * (DK / 4);
-            const size_t src = ((size_t)(cs + (i < Cn ? i : 0)) * nk + kh) * DK;
-            rk[m] = ldg((const float4 *)(kn + src) + c);
-            rq[m] = ldg((const float4 *)(qn + src) + c);
-        }
-        const float *gm = grams + ((size_t)chn * nk + kh) * 2 * CH * CH;
-#pragma unroll
-        for (int m = 0; m < NG; m++) {
-            rm[m] = ldg(gm + tid + 256 * m);
-            rw[m] = ldg(gm + CH * CH + tid + 256 * m);
-        }
-        if (tid < Cn) {
-            ral = ldg(al + (size_t)(cs + tid) * nv + hv);
-            rbe = ldg(be + (size_t)(cs + tid) * nv + hv);
-        }
-#pragma unroll
-        for (int m = 0; m < NU; m++) {
-            const int e = tid + 256 * m, i = e / RB, rr = e - i * RB;
-            ru[m] = ldg(conv + (size_t)(cs + (i < Cn ? i : 0)) * cc + 2 * qd + r0 + rr);
-        }
-    };
-    fetch(0, 0);
-    for (int c0 = 0, ch = 0; c0 < T; c0 += CH, ch++) {
-        const int C = T - c0 < CH ? T - c0 : CH;
-        __syncthreads();                                 // the previous chunk is consumed
-#pragma unroll
-        for (int m = 0; m < NKQ; m++) {
-            const int e = tid + 256 * m, i = e / (DK / 4), c = e - i * (DK / 4);
-            if (i < C) {
-                *(float4 *)(&kc[i][4 * c]) = rk[m];
-                *(float4 *)(&qc[i][4 * c]) = rq[m];
-            }
-        }
-#pragma unroll
-        for (int m = 0; m < NG; m++) {
-            const int e = tid + 256 * m;
-            M[e / CH][e % CH] = rm[m];
-            W[e / CH][e % CH] = rw[m];
-        }
-        if (tid < C) {
-            alpha[tid] = ral;
-            beta[tid] = rbe;
-        }
-#pragma unroll
-        for (int m = 0; m < NU; m++) {
-            const int e = tid + 256 * m, i = e / RB, rr = e - i * RB;
-            if (i < C) U[i][rr] = ru[m];
-        }
-        fetch(c0 + CH, ch + 1);
-        __syncthreads();
-        // decay products: thread i owns row i of the coefficient tables, which
-        // turn in place into M[i][j] = beta_i (p_i/p_j) k_j.k_i and
-        // W[i][j] = (p_i/p_j) k_j.q_i
-        // (the gates and row i are read into registers first, so the
-        // product chains wait on no LDS read; the same products in the same
-        // order as a loop over LDS)
-        if (tid < C) {
-            const int i = tid;
-            float ag[CH], mr[CH], wr[CH];
-#pragma unroll
-            for (int l = 0; l < CH; l++) ag[l] = alpha[l];
-#pragma unroll
-            for (int q = 0; q < CH / 4; q++) {
-                const float4 vm = *(const float4 *)&M[i][4 * q], vw = *(const float4 *)&W[i][4 * q];
-                mr[4 * q] = vm.x; mr[4 * q + 1] = vm.y; mr[4 * q + 2] = vm.z; mr[4 * q + 3] = vm.w;
-                wr[4 * q] = vw.x; wr[4 * q + 1] = vw.y; wr[4 * q + 2] = vw.z; wr[4 * q + 3] = vw.w;
-            }
-            float pi = ag[0];
-#pragma unroll
-            for (int l = 1; l < CH; l++)
-                if (l <= i) pi = pi * ag[l];
-            p[i] = pi;
-            const float bi = beta[i];
-            float ratio = 1.0f;
-            int z = 0;
-#pragma unroll
-            for (int j = CH - 2; j >= 0; j--) {
-                if (j < i) {
-                    ratio *= ag[j + 1];
-                    const float mij = bi * ratio * mr[j];
-                    mr[j] = mij;
-                    z |= mij == 0.0f;
-                    wr[j] = ratio * wr[j];
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < CH / 4; q++) {
-                *(float4 *)&M[i][4 * q] = float4{mr[4 * q], mr[4 * q + 1], mr[4 * q + 2], mr[4 * q + 3]};
-                *(float4 *)&W[i][4 * q] = float4{wr[4 * q], wr[4 * q + 1], wr[4 * q + 2], wr[4 * q + 3]};
-            }
-            mz[i] = z;
-        }
-        if (tid == 64) {
-            float ag[CH];
-#pragma unroll
-            for (int l = 0; l < CH; l++) ag[l] = alpha[l];
-            float ratio = 1.0f;
-#pragma unroll
-            for (int j = CH - 1; j >= 0; j--) {
-                if (j < C) {
-                    wend[j] = ratio;
-                    ratio *= ag[j];
-                }
-            }
-        }
-        __syncthreads();
-        // projections of the incoming state, tokens g and g + 16; U starts as
-        // t_i = beta_i v_i - beta_i p_i (S_in k_i); the state row comes from
-        // LDS here (it is live only in this phase)
-        reload();
-        {
-            const int i0 = g, i1 = g + RB;
-            const int j0 = i0 < C ? i0 : 0, j1 = i1 < C ? i1 : 0;
-            float ak0 = 0.0f, aq0 = 0.0f, ak1 = 0.0f, aq1 = 0.0f;
-#pragma unroll
-            for (int c = 0; c < DK; c++) {
-                ak0 += s[c] * kc[j0][c];
-                aq0 += s[c] * qc[j0][c];
-                ak1 += s[c] * kc[j1][c];
-                aq1 += s[c] * qc[j1][c];
-            }
-            if (i0 < C) {
-                U[i0][r] = beta[i0] * U[i0][r] - beta[i0] * p[i0] * ak0;
-                Sq[i0][r] = aq0;
-            }
-            if (i1 < C) {
-                U[i1][r] = beta[i1] * U[i1][r] - beta[i1] * p[i1] * ak1;
-                Sq[i1][r] = aq1;
-            }
-        }
-        __syncthreads();
-        // forward substitution (I + M) U = T, a thread per row, in registers:
-        // u_i = (((t_i - m_{i,i-1} u_{i-1}) - m_{i,i-2} u_{i-2}) ...), a term
-        // with m = 0 skipped (subtracting an exact +0 leaves u_i's bits as
-        // they are, so the zero test sits on the product, off the chain). Row
-        // i's coefficients are read into registers before its chain starts.
-        if (tid < RB) {
-            float u[CH];
-#pragma unroll
-            for (int i = 0; i < CH; i++) u[i] = i < C ? U[i][tid] : 0.0f;
-#pragma unroll
-            for (int i = 1; i < CH; i++) {
-                if (i < C) {
-                    float mr[CH];
-#pragma unroll
-                    for (int q = 0; q < CH / 4; q++)
-                        if (4 * q < i) {
-                            const float4 v = *(const float4 *)&M[i][4 * q];
-                            mr[4 * q] = v.x; mr[4 * q + 1] = v.y; mr[4 * q + 2] = v.z; mr[4 * q + 3] = v.w;
-                        }
-                    float ui = u[i];
-                    if (__builtin_amdgcn_readfirstlane(mz[i]) == 0) {
-#pragma unroll
-                        for (int j = i - 1; j >= 0; j--) ui = ui - mr[j] * u[j];
-                    } else {
-#pragma unroll
-                        for (int j = i - 1; j >= 0; j--) {
-                            const float pr = mr[j] != 0.0f ? mr[j] * u[j] : 0.0f;
-                            ui = ui - pr;
-                        }
-                    }
-                    u[i] = ui;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < CH; i++)
-                if (i < C) U[i][tid] = u[i];
-        }
-        __syncthreads();
-        // outputs of tokens g and g + 16, scaled by 1/sqrt(dk): o_i =
-        // p_i Sq_i + w_ii u_i + sum_{j<i} w_ij u_j, j descending
-        {
-            float u[CH];
-#pragma unroll
-            for (int j = 0; j < CH; j++) u[j] = j < C ? U[j][r] : 0.0f;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int i = g + RB * h;
-                if (i < C) {
-                    float wr[CH];
-#pragma unroll
-                    for (int q = 0; q < CH / 4; q++) {
-                        const float4 v = *(const float4 *)&W[i][4 * q];
-                        wr[4 * q] = v.x; wr[4 * q + 1] = v.y; wr[4 * q + 2] = v.z; wr[4 * q + 3] = v.w;
-                    }
-                    float o = p[i] * Sq[i][r];
-                    o += W[i][i] * U[i][r];
-#pragma unroll
-                    for (int j = CH - 1; j >= 0; j--)
-                        if (j < i) o += wr[j] * u[j];
-                    o *= out_scale;
-                    stg(out + (size_t)(c0 + i) * vd + r0 + r, o);
-                }
-            }
-        }
-        // S_out = p_{C-1} S_in + sum_j (p_{C-1}/p_j) u_j k_j^T, j descending:
-        // CPL columns of row ur
-        {
-            const float pc = p[C - 1];
-            float x[CPL], uw[CH];
-            float *xr = xs + ur * XS + ucg * CPL;
-#pragma unroll
-            for (int j = 0; j < CH; j++) uw[j] = j < C ? wend[j] * U[j][ur] : 0.0f;
-#pragma unroll
-            for (int c = 0; c < CPL; c++) x[c] = xr[c] * pc;
-#pragma unroll
-            for (int j = CH - 1; j >= 0; j--) {
-                if (j < C) {
-                    // the key segment is read whether or not the term is
-                    // skipped, so the reads can run ahead of the sums
-                    float kk[CPL];
-#pragma unroll
-                    for (int c4 = 0; c4 < CPL / 4; c4++) {
-                        const float4 v = *(const float4 *)&kc[j][ucg * CPL + 4 * c4];
-                        kk[4 * c4] = v.x; kk[4 * c4 + 1] = v.y; kk[4 * c4 + 2] = v.z; kk[4 * c4 + 3] = v.w;
-                    }
-                    const float uj = uw[j];
-                    if (uj != 0.0f) {
-#pragma unroll
-                        for (int c = 0; c < CPL; c++) x[c] += uj * kk[c];
-                    }
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < CPL; c++) xr[c] = x[c];
-        }
-    }
-    __syncthreads();                                     // every row's update is in LDS
-    for (int e = tid; e < RB * DK / 4; e += 256) {
-        const int row = e / (DK / 4), c4 = e - row * (DK / 4);
-        stg((float4 *)Srow + e, *(const float4 *)(xs + row * XS + 4 * c4));
-    }
 }
 
 // ---- gated per-head RMSNorm + Q8_K of T vectors (src/ornith_rforward.c:300-319) ---
