@@ -66,6 +66,20 @@ bool pf_moe_slots_ok(const OhLayer &y) {
     return true;
 }
 
+// IQ2_XXS experts of at least this many (token, expert) slots run grouped by
+// expert, the weights formed once for up to cols slots; fewer slots keep the
+// token step's rows (a launch per slot and row, shorter chains). 512 experts,
+// top 10, gate/up 4096 -> 1024, one layer, a whole request in us, rows per slot
+// against groups of 4 and of 8: 400 slots 2038 / 2017 / 2263, 1280: 4604 / 4242 /
+// 4417, 2000: 7077 / 6169 / 6028, 5000: 15692 / 11513 / 10802
+constexpr int kIq2MinSlots = 480;
+bool pf_iq2_slots(const ornith_hip_tensor *W, int slots) {
+    return W->type == OH_IQ2_XXS && !iq2_tree_on() && slots >= kIq2MinSlots;
+}
+int pf_iq2_cols(int n) { return n < 1800 ? 4 : 8; }
+// the most pieces of up to pf_iq2_cols slots of one expert that n slots make
+int pf_iq2_items(int n, int ne) { return n / pf_iq2_cols(n) + (ne < n ? ne : n); }
+
 bool pf_supported(const ornith_hip_model *m) {
     const ornith_hip_arch &a = m->a;
     if (a.hidden > 8192 || a.nv * a.dv > 8192 || a.nh * a.hd > 8192) return false;
@@ -122,12 +136,12 @@ int pf_alloc(ornith_hip_session *s, int tc) {
     CHK(salloc(s, &p.FPML, (size_t)kPfAttnSub * a.nh * nch * 2 + 64));
     CHK(salloc(s, &p.RL, T * ne)); CHK(salloc(s, &p.SHL, T)); CHK(salloc(s, &p.SHG, T));
     CHK(salloc(s, &p.RW, T * K)); CHK(salloc(s, &p.RIDX, T * K));
-    CHK(salloc(s, &p.CNT, ne)); CHK(salloc(s, &p.LIST, ne * T));
+    CHK(salloc(s, &p.CNT, ne + 1)); CHK(salloc(s, &p.LIST, ne * T));
     CHK(salloc(s, &p.Hh, T * K * I)); CHK(q8alloc(s, p.HQ, T * K * I + 256));
     CHK(salloc(s, &p.HSH, T * sI)); CHK(q8alloc(s, p.HSQ, T * sI + 256));
     CHK(salloc(s, &p.OD, T * K * H)); CHK(salloc(s, &p.ODSH, T * H));
     CHK(salloc(s, &p.GU, T * K * 2 * I)); CHK(salloc(s, &p.GSH, T * 2 * sI));
-    CHK(salloc(s, &p.ITEMS, (T * K + 63) / 64 + ne + 2));
+    CHK(salloc(s, &p.ITEMS, (T * K + 3) / 4 + ne + 2));   // pieces of 64 columns, or of 4 or 8 (pf_iq2_cols)
     CHK(salloc(s, &p.XN, T * H));
     p.tc = tc;
     p.WY = nullptr;                       // sized for tc tokens on its first use
@@ -307,26 +321,43 @@ int pf_chunk(ornith_hip_session *s, int base, int T, bool chunked, hipStream_t s
                 // token t's j-th routed expert and reads token t's normalised
                 // row (and Q8_K planes) or its own silu(gate) * up
                 const Act ax = act_of(p.XQ, p.XN);
-                MvBuild b2, b3;
-                if (pairable(y.gate_exps, y.up_exps)) {
+                const bool gu = pf_iq2_slots(y.gate_exps, T * K) && pf_iq2_slots(y.up_exps, T * K) &&
+                                y.up_exps->rows == y.gate_exps->rows && y.up_exps->in == y.gate_exps->in;
+                const bool dn = (gu || pairable(y.gate_exps, y.up_exps)) && pf_iq2_slots(y.down_exps, T * K);
+                const int cols = pf_iq2_cols(T * K), slot_items = pf_iq2_items(T * K, a.ne);
+                if (gu || dn) HCHK(oh_launch_slot_lists(p.RIDX, T * K, a.ne, cols, p.CNT, p.LIST, p.ITEMS, st));
+                Act ah;
+                ah.pro = OH_PRO_F32;
+                ah.xf = p.Hh;
+                if (gu) {
+                    oh_iq2rows R = {y.gate_exps->A, y.gate_exps->C, y.up_exps->A, y.up_exps->C, p.XN, p.Hh, p.CNT, p.LIST,
+                                    p.ITEMS, H, I, H, I, K, cols};
+                    HCHK(oh_launch_iq2_slots(&R, slot_items, st));
+                } else if (pairable(y.gate_exps, y.up_exps)) {
+                    MvBuild b2;
                     CHK(mv_add_pair(b2, y.gate_exps, y.up_exps, ax, p.Hh, p.RIDX, T * K, I));
                     b2.L.s[b2.L.n - 1].astride = H;
                     b2.L.s[b2.L.n - 1].adiv = K;
                     CHK(mv_go(b2, st));
-                    Act ah;
-                    ah.pro = OH_PRO_F32;
-                    ah.xf = p.Hh;
-                    CHK(mv_add(b3, y.down_exps, ah, p.OD, 0, p.RIDX, T * K, H, I));
                 } else {
+                    MvBuild b2;
                     float *G = p.GU, *U = p.GU + (size_t)T * K * I;
                     CHK(mv_add(b2, y.gate_exps, ax, G, 0, p.RIDX, T * K, I, H));
                     b2.L.s[b2.L.n - 1].adiv = K;
                     CHK(mv_add(b2, y.up_exps, ax, U, 0, p.RIDX, T * K, I, H));
                     b2.L.s[b2.L.n - 1].adiv = K;
                     CHK(mv_go(b2, st));
-                    CHK(mv_add(b3, y.down_exps, act_swiglu(G, U), p.OD, 0, p.RIDX, T * K, H, I));
+                    ah = act_swiglu(G, U);
                 }
-                CHK(mv_go(b3, st));
+                if (dn) {
+                    oh_iq2rows R = {y.down_exps->A, y.down_exps->C, nullptr, nullptr, p.Hh, p.OD, p.CNT, p.LIST, p.ITEMS,
+                                    I, H, I, H, 1, cols};
+                    HCHK(oh_launch_iq2_slots(&R, slot_items, st));
+                } else {
+                    MvBuild b3;
+                    CHK(mv_add(b3, y.down_exps, ah, p.OD, 0, p.RIDX, T * K, H, I));
+                    CHK(mv_go(b3, st));
+                }
             } else {
                 HCHK(oh_launch_group_pairs(p.RIDX, T * K, p.CNT, a.ne, p.LIST, T, s->io + OH_IO_ERR, st));
                 const int max_items = (T * K + 63) / 64 + a.ne;

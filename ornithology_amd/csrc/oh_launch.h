@@ -59,6 +59,13 @@ bool oh_mmq_can(uint32_t type, int rows, int in);
 // `rows` rows (a multiple of 64) from its A and B planes
 hipError_t oh_launch_mmq_tiles(const uint8_t *A, const uint8_t *B, uint8_t *PA, uint8_t *PB, int64_t rows,
                                int nb, int P, hipStream_t st);
+// a chunk's IQ2_XXS experts: the slots grouped by expert (ne <= 1024; off: ne + 1
+// entries, list: n, items: those of up to cols (<= 8) slots each,
+// after their count), then
+// the rows of every expert over its slots
+hipError_t oh_launch_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32_t *list, int32_t *items,
+                                hipStream_t st);
+hipError_t oh_launch_iq2_slots(const oh_iq2rows *a, int max_items, hipStream_t st);
 // decode of n sessions at once: the decode bodies, one grid row per session,
 // descriptors and positions in device arrays of n
 hipError_t oh_launch_delta_batch(const oh_op_delta *ops, const int32_t *pos, int n, int dk, int K, int nv,

@@ -312,6 +312,17 @@ typedef struct {
     } u;
 } oh_op;
 
+// IQ2_XXS rows over the slots of a chunk, grouped by expert (off, list and
+// items of oh_launch_slot_lists, up to cols slots of one expert an item): slot p reads activation row p / adiv and writes output
+// row p; with A2/C2 (gate and up) the output is silu(A . x) * (A2 . x)
+typedef struct {
+    const uint8_t *A, *C, *A2, *C2;
+    const float *x;
+    float *y;
+    const int32_t *off, *list, *items;
+    int in, rows, xstride, ystride, adiv, cols;
+} oh_iq2rows;
+
 // Persistent step kernel: counters of one program phase (one per 64-byte
 // line, OH_STEP_NCTR of them) and the io words it uses.
 #define OH_STEP_NCTR 32

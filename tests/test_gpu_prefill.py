@@ -215,3 +215,28 @@ def test_mfma_prompt_attention_within_tolerance(hip_ctx, orc, tmp_path, monkeypa
         assert int(np.argmax(got)) == int(np.argmax(want)), mfma
         s.free()
     m.free()
+
+
+@pytest.mark.parametrize("ne,top_k,n", [(8, 2, 239), (8, 2, 240), (8, 2, 451), (32, 4, 163), (32, 4, 449), (32, 4, 512)])
+def test_iq2_experts_grouped_equal_token_path(hip_ctx, monkeypatch, ne, top_k, n):
+    """IQ2_XXS experts around the slot counts (480, 1800) where the prompt starts
+    to group its (token, expert) slots by expert and to walk eight of them
+    together, with remainders of every size, then a second, shorter prompt in
+    the same session's buffers: logits and session state bit-identical to the
+    token-by-token path."""
+    m = hip_ctx.synth(**dict(IQ2X, n_layers=2, full_interval=2, ne=ne, top_k=top_k, seed=17))
+    p = np.random.default_rng(n).integers(0, m.arch["vocab"], n).astype(np.int32)
+    got = []
+    for prefill in ("1", "0"):
+        monkeypatch.setenv("ORNITH_HIP_PREFILL", prefill)
+        s = m.session(2 * n)
+        s.eval(p)
+        first = s.logits().copy()
+        s.eval(p[:n * 4 // 5])
+        got.append((s, first, s.logits().copy()))
+    assert np.array_equal(u32(got[0][1]), u32(got[1][1]))
+    assert np.array_equal(u32(got[0][2]), u32(got[1][2]))
+    same_state(m, got[0][0], got[1][0])
+    for s, _, _ in got:
+        s.free()
+    m.free()
