@@ -67,12 +67,27 @@ void seterr(const char *fmt, ...);
 
 
 // ---- context -----------------------------------------------------------------------
+// One device allocation of the context's pool (dev_get / dev_put).
+struct DevBlock { void *p = nullptr; size_t n = 0; };
+
 struct ornith_hip_ctx {
     int device = 0;
     hipStream_t st = nullptr;
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    // allocations of closed sessions, kept for the next ones: work on them is
+    // ordered by the context's one stream
+    std::mutex pool_mu;
+    std::vector<DevBlock> pool;
+    size_t pool_bytes = 0;
 };
+// hipMalloc that gives the pool's blocks back and tries again when memory is short
+hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n);
+// a block of at least n bytes (contents undefined) from the pool or the device
+hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b);
+// the block back to the pool, or to the device beyond kPoolBytes
+void dev_put(ornith_hip_ctx *c, const DevBlock &b);
+void dev_trim(ornith_hip_ctx *c);
 
 // ---- tensors in the plane layout (oh_types.h) ---------------------------------------
 struct ornith_hip_tensor {
@@ -137,6 +152,12 @@ struct ornith_hip_model {
     bool any_full = false;        // a full-attention (GQA) layer exists
     ornith_hip_tensor *embd = nullptr, *out_norm = nullptr, *lm_head = nullptr;
     uint64_t bytes = 0;
+    // RoPE (cos, sin) of positions < rope_cap, shared by the model's sessions;
+    // the tables it outgrew stay until the model is freed
+    std::mutex rope_mu;
+    float2 *rope = nullptr;
+    int rope_cap = 0;
+    std::vector<float2 *> rope_all;
 };
 
 // metadata view shared by the GGUF and synthetic paths
@@ -165,8 +186,13 @@ struct ornith_hip_session {
     uint64_t sid = 0;             // unique per session of the process
     int cap = 0, pos = 0, kvcap = 0;
     bool have_logits = false;
-    std::vector<void *> allocs;
+    std::vector<void *> allocs;   // the session's buffers, parts of its blocks (and the RoPE table)
     std::vector<size_t> asz;      // bytes requested for each of allocs
+    std::vector<DevBlock> blocks; // device memory the session holds
+    char *cur = nullptr;          // the last block's free part
+    size_t left = 0;
+    bool measuring = false;       // salloc adds up sizes only
+    size_t need = 0;
     int32_t *io = nullptr;        // [0] pos, [1] best
     int32_t *toks = nullptr;      // [cap + 1]
     float *x = nullptr, *xn = nullptr;
@@ -285,15 +311,34 @@ struct Prog {
     bool step = false;            // built for the persistent step kernel
 };
 
+// a zeroed block of n bytes for the session's next buffers
+int sreserve(ornith_hip_session *s, size_t n);
+// n elements of the session's memory, zeroed, with 256 bytes after them
 template <typename T>
 static int salloc(ornith_hip_session *s, T **p, size_t n) {
-    void *v = nullptr;
-    HCHK(hipMalloc(&v, n * sizeof(T) + 256));
-    HCHK(hipMemset(v, 0, n * sizeof(T) + 256));
-    s->allocs.push_back(v);
+    const size_t bytes = (n * sizeof(T) + 256 + 255) & ~(size_t)255;
+    if (s->measuring) { s->need += bytes; return ORNITH_HIP_OK; }
+    if (bytes > s->left) {
+        const int r = sreserve(s, bytes);
+        if (r != ORNITH_HIP_OK) return r;
+    }
+    s->allocs.push_back(s->cur);
     s->asz.push_back(n * sizeof(T));
-    *p = (T *)v;
+    *p = (T *)s->cur;
+    s->cur += bytes;
+    s->left -= bytes;
     return ORNITH_HIP_OK;
+}
+// lay(): a sequence of salloc calls, run once to add up their sizes and once
+// over one block of that size
+template <typename F>
+static int slayout(ornith_hip_session *s, F &&lay) {
+    s->measuring = true;
+    s->need = 0;
+    int r = lay();
+    s->measuring = false;
+    if (r == ORNITH_HIP_OK) r = sreserve(s, s->need);
+    return r == ORNITH_HIP_OK ? lay() : r;
 }
 
 struct DecB {

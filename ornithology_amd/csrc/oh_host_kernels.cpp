@@ -51,7 +51,7 @@ int mmq_tiles(const ornith_hip_tensor *W, hipStream_t st) {
     }
     const size_t nblk = (size_t)W->rows * (size_t)(W->in / 256), a = nblk * 16 * P, b = nblk * 16;
     uint8_t *mem = nullptr;
-    hipError_t e = hipMalloc(&mem, up256(a) + b);
+    hipError_t e = dev_malloc(W->ctx, (void **)&mem, up256(a) + b);
     if (e != hipSuccess) {
         seterr("tensor '%s': prompt tiles, hipMalloc(%zu): %s", W->name.c_str(), up256(a) + b,
                hipGetErrorString(e));
@@ -189,19 +189,33 @@ extern "C" int ornith_hip_quantize(ornith_hip_ctx *ctx, uint32_t type, const flo
     }
     if (n == 0 || n % 256) { seterr("quantize: %llu values is not a whole number of 256-blocks", (unsigned long long)n); return ORNITH_HIP_ERR_FORMAT; }
     HCHK(hipSetDevice(ctx->device));
-    const uint64_t dims[2] = {256, n / 256};
-    ornith_hip_tensor *t = nullptr;
-    CHK(tensor_alloc(ctx, "quantize", type, 2, dims, &t));
-    float *dx = nullptr;
-    hipError_t e = hipMalloc(&dx, n * 4);
-    if (e == hipSuccess) e = hipMemcpyAsync(dx, x, n * 4, hipMemcpyHostToDevice, ctx->st);
-    if (e == hipSuccess) e = oh_launch_encode(dx, (int)type, (int64_t)(n / 256), t->A, t->B, t->C, ctx->st);
+    // the planes and the values in one block of the pool
+    ornith_hip_tensor t;
+    t.ctx = ctx;
+    t.name = "quantize";
+    t.type = type;
+    t.nd = 2;
+    t.dims[0] = 256;
+    t.dims[1] = n / 256;
+    t.in = 256;
+    t.rows = (int64_t)(n / 256);
+    t.gguf_bytes = gguf_nbytes(type, n);
+    size_t pa, pb, pc;
+    plane_bytes(type, t.rows, t.in, &pa, &pb, &pc);
+    DevBlock blk;
+    hipError_t e = dev_get(ctx, up256(pa) + up256(pb) + up256(pc) + n * 4, &blk);
+    if (e != hipSuccess) { seterr("quantize: %s", hipGetErrorString(e)); return ORNITH_HIP_ERR_OOM; }
+    t.mem = t.A = (uint8_t *)blk.p;
+    t.B = t.A + up256(pa);
+    t.C = t.B + up256(pb);
+    float *dx = (float *)(t.C + up256(pc));
+    e = hipMemcpyAsync(dx, x, n * 4, hipMemcpyHostToDevice, ctx->st);
+    if (e == hipSuccess) e = oh_launch_encode(dx, (int)type, (int64_t)(n / 256), t.A, t.B, t.C, ctx->st);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->st);
-    if (dx) (void)hipFree(dx);
     int r = ORNITH_HIP_OK;
     if (e != hipSuccess) { seterr("quantize: %s", hipGetErrorString(e)); r = ORNITH_HIP_ERR_DEVICE; }
-    if (r == ORNITH_HIP_OK) r = ornith_hip_tensor_download(t, out, t->gguf_bytes);
-    ornith_hip_tensor_free(t);
+    if (r == ORNITH_HIP_OK) r = ornith_hip_tensor_download(&t, out, t.gguf_bytes);
+    dev_put(ctx, blk);
     return r;
 }
 

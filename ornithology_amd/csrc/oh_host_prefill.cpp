@@ -117,32 +117,35 @@ int pf_alloc(ornith_hip_session *s, int tc) {
     const size_t K = a.top_k > 0 ? a.top_k : 1, I = a.moe_inter > 0 ? a.moe_inter : 1;
     const size_t sI = a.shared_inter > 0 ? a.shared_inter : 1, ne = a.ne > 0 ? a.ne : 1;
     const size_t nch = (s->kvcap + oh_flash_chunk() - 1) / oh_flash_chunk();
-    CHK(salloc(s, &p.X, T * H));
-    CHK(q8alloc(s, p.XQ, T * H));
-    const size_t T32 = (T + 31) / 32 * 32;   // the delta scan reads whole 32-token chunks
-    CHK(salloc(s, &p.CAT, T * cc + 1)); CHK(salloc(s, &p.CONV, T32 * cc + 1));
-    CHK(salloc(s, &p.Z, T * vd + 1)); CHK(salloc(s, &p.O, T * vd + 1));
-    CHK(q8alloc(s, p.OQ, T * vd + 256));
-    CHK(salloc(s, &p.A, T * a.nv + 1)); CHK(salloc(s, &p.Bg, T * a.nv + 1));
-    CHK(salloc(s, &p.AL, T * a.nv + 1)); CHK(salloc(s, &p.BE, T * a.nv + 1));
-    CHK(salloc(s, &p.QN, T32 * qd + 1)); CHK(salloc(s, &p.KN, T32 * qd + 1));
-    const int gr = oh_delta_grams_floats(tc, a.nk > 0 ? a.nk : 1), co = oh_delta_coef_floats(tc, a.nv > 0 ? a.nv : 1);
-    CHK(salloc(s, &p.GR, (size_t)(gr > co ? gr : co) + 1));
-    CHK(salloc(s, &p.STAGE, (size_t)(a.conv_k > 1 ? a.conv_k - 1 : 1) * cc + 1));
-    CHK(salloc(s, &p.QP, T * 2 * aq + 1)); CHK(salloc(s, &p.KB, T * kvd + 1)); CHK(salloc(s, &p.VB, T * kvd + 1));
-    CHK(salloc(s, &p.QR, T * aq + 1)); CHK(salloc(s, &p.AG, T * aq + 1)); CHK(salloc(s, &p.OA, T * aq + 1));
-    CHK(q8alloc(s, p.OAQ, T * aq + 256));
-    CHK(salloc(s, &p.FPO, (size_t)kPfAttnSub * a.nh * nch * a.hd + 64));
-    CHK(salloc(s, &p.FPML, (size_t)kPfAttnSub * a.nh * nch * 2 + 64));
-    CHK(salloc(s, &p.RL, T * ne)); CHK(salloc(s, &p.SHL, T)); CHK(salloc(s, &p.SHG, T));
-    CHK(salloc(s, &p.RW, T * K)); CHK(salloc(s, &p.RIDX, T * K));
-    CHK(salloc(s, &p.CNT, ne + 1)); CHK(salloc(s, &p.LIST, ne * T));
-    CHK(salloc(s, &p.Hh, T * K * I)); CHK(q8alloc(s, p.HQ, T * K * I + 256));
-    CHK(salloc(s, &p.HSH, T * sI)); CHK(q8alloc(s, p.HSQ, T * sI + 256));
-    CHK(salloc(s, &p.OD, T * K * H)); CHK(salloc(s, &p.ODSH, T * H));
-    CHK(salloc(s, &p.GU, T * K * 2 * I)); CHK(salloc(s, &p.GSH, T * 2 * sI));
-    CHK(salloc(s, &p.ITEMS, (T * K + 3) / 4 + ne + 2));   // pieces of 64 columns, or of 4 or 8 (pf_iq2_cols)
-    CHK(salloc(s, &p.XN, T * H));
+    CHK(slayout(s, [&]() -> int {
+        CHK(salloc(s, &p.X, T * H));
+        CHK(q8alloc(s, p.XQ, T * H));
+        const size_t T32 = (T + 31) / 32 * 32;   // the delta scan reads whole 32-token chunks
+        CHK(salloc(s, &p.CAT, T * cc + 1)); CHK(salloc(s, &p.CONV, T32 * cc + 1));
+        CHK(salloc(s, &p.Z, T * vd + 1)); CHK(salloc(s, &p.O, T * vd + 1));
+        CHK(q8alloc(s, p.OQ, T * vd + 256));
+        CHK(salloc(s, &p.A, T * a.nv + 1)); CHK(salloc(s, &p.Bg, T * a.nv + 1));
+        CHK(salloc(s, &p.AL, T * a.nv + 1)); CHK(salloc(s, &p.BE, T * a.nv + 1));
+        CHK(salloc(s, &p.QN, T32 * qd + 1)); CHK(salloc(s, &p.KN, T32 * qd + 1));
+        const int gr = oh_delta_grams_floats(tc, a.nk > 0 ? a.nk : 1), co = oh_delta_coef_floats(tc, a.nv > 0 ? a.nv : 1);
+        CHK(salloc(s, &p.GR, (size_t)(gr > co ? gr : co) + 1));
+        CHK(salloc(s, &p.STAGE, (size_t)(a.conv_k > 1 ? a.conv_k - 1 : 1) * cc + 1));
+        CHK(salloc(s, &p.QP, T * 2 * aq + 1)); CHK(salloc(s, &p.KB, T * kvd + 1)); CHK(salloc(s, &p.VB, T * kvd + 1));
+        CHK(salloc(s, &p.QR, T * aq + 1)); CHK(salloc(s, &p.AG, T * aq + 1)); CHK(salloc(s, &p.OA, T * aq + 1));
+        CHK(q8alloc(s, p.OAQ, T * aq + 256));
+        CHK(salloc(s, &p.FPO, (size_t)kPfAttnSub * a.nh * nch * a.hd + 64));
+        CHK(salloc(s, &p.FPML, (size_t)kPfAttnSub * a.nh * nch * 2 + 64));
+        CHK(salloc(s, &p.RL, T * ne)); CHK(salloc(s, &p.SHL, T)); CHK(salloc(s, &p.SHG, T));
+        CHK(salloc(s, &p.RW, T * K)); CHK(salloc(s, &p.RIDX, T * K));
+        CHK(salloc(s, &p.CNT, ne + 1)); CHK(salloc(s, &p.LIST, ne * T));
+        CHK(salloc(s, &p.Hh, T * K * I)); CHK(q8alloc(s, p.HQ, T * K * I + 256));
+        CHK(salloc(s, &p.HSH, T * sI)); CHK(q8alloc(s, p.HSQ, T * sI + 256));
+        CHK(salloc(s, &p.OD, T * K * H)); CHK(salloc(s, &p.ODSH, T * H));
+        CHK(salloc(s, &p.GU, T * K * 2 * I)); CHK(salloc(s, &p.GSH, T * 2 * sI));
+        CHK(salloc(s, &p.ITEMS, (T * K + 3) / 4 + ne + 2));   // pieces of 64 columns, or of 4 or 8 (pf_iq2_cols)
+        CHK(salloc(s, &p.XN, T * H));
+        return ORNITH_HIP_OK;
+    }));
     p.tc = tc;
     p.WY = nullptr;                       // sized for tc tokens on its first use
     return ORNITH_HIP_OK;

@@ -68,7 +68,7 @@ extern "C" void ornith_hip_session_free(ornith_hip_session *s) {
     if (s->gbody_x) (void)hipGraphExecDestroy(s->gbody_x);
     if (s->ghead) (void)hipGraphExecDestroy(s->ghead);
     if (s->bw.graph) (void)hipGraphExecDestroy(s->bw.graph);
-    for (void *p : s->allocs) (void)hipFree(p);
+    for (const DevBlock &b : s->blocks) dev_put(s->m->ctx, b);
     delete s;
 }
 int q8alloc(ornith_hip_session *s, Q8Buf &q, size_t n) {
@@ -94,6 +94,48 @@ Act act_swiglu(const float *g, const float *u) {
     Act a; a.pro = OH_PRO_SWIGLU; a.xf = g; a.xf2 = u; return a;
 }
 
+// RoPE cos/sin per (position, pair) with the reference's libm calls
+// (ot_rope_partial, src/ornith_tensor.c:167-178), once per model: a longer
+// session's table replaces it, half again as long at least
+static int rope_table(ornith_hip_model *m, ornith_hip_session *s) {
+    const ornith_hip_arch &a = m->a;
+    const int half = a.hd / 2;
+    std::lock_guard<std::mutex> lk(m->rope_mu);
+    if (s->cap > m->rope_cap) {
+        int rot = a.rope_dim;
+        if (rot <= 0 || rot > a.hd) rot = a.hd;
+        const int cap = s->cap > m->rope_cap + m->rope_cap / 2 ? s->cap : m->rope_cap + m->rope_cap / 2;
+        std::vector<float2> tab((size_t)cap * half);
+        std::vector<float> freq((size_t)rot / 2);
+        for (int i = 0; i < rot / 2; i++) freq[i] = powf(a.rope_theta, -2.0f * (float)i / (float)rot);
+        for (int p = 0; p < cap; p++)
+            for (int i = 0; i < half; i++) {
+                float2 cs = {1.0f, 0.0f};
+                if (i < rot / 2) {
+                    const float ang = (float)p * freq[i];
+                    cs.x = cosf(ang);
+                    cs.y = sinf(ang);
+                }
+                tab[(size_t)p * half + i] = cs;
+            }
+        float2 *d = nullptr;
+        HCHK(dev_malloc(m->ctx, (void **)&d, tab.size() * sizeof(float2) + 256));
+        const hipError_t e = hipMemcpy(d, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(d);
+            seterr("rope upload: %s", hipGetErrorString(e));
+            return ORNITH_HIP_ERR_DEVICE;
+        }
+        m->rope_all.push_back(d);
+        m->rope = d;
+        m->rope_cap = cap;
+    }
+    s->rope = m->rope;
+    s->allocs.push_back(s->rope);
+    s->asz.push_back((size_t)m->rope_cap * half * sizeof(float2));
+    return ORNITH_HIP_OK;
+}
+
 extern "C" int ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_session **out) {
     *out = nullptr;
     if (cap < 1) cap = 1;
@@ -109,88 +151,69 @@ extern "C" int ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_s
     const int aq = a.nh * a.hd, kvd = a.nkv * a.hd;
     const int K = a.top_k, I = a.moe_inter > a.shared_inter ? a.moe_inter : a.shared_inter;
     const int ow = vd > aq ? vd : aq;
-    int st = ORNITH_HIP_OK;
-#define A_(x) do { if ((st = (x)) != ORNITH_HIP_OK) { ornith_hip_session_free(s); return st; } } while (0)
-    A_(salloc(s, &s->io, 64));
-    A_(salloc(s, &s->toks, (size_t)cap + 1));
-    A_(salloc(s, &s->x, H)); A_(salloc(s, &s->xn, H)); A_(q8alloc(s, s->xq, H));
-    A_(salloc(s, &s->cat, cc > 0 ? cc : 1)); A_(salloc(s, &s->gate, vd > 0 ? vd : 1));
-    A_(salloc(s, &s->ab, 2 * (a.nv > 0 ? a.nv : 1)));
-    A_(salloc(s, &s->o, ow)); A_(q8alloc(s, s->oq, ow));
-    A_(salloc(s, &s->qproj, 2 * (size_t)aq)); A_(salloc(s, &s->kb, kvd)); A_(salloc(s, &s->vb, kvd));
-    A_(salloc(s, &s->qr, aq)); A_(salloc(s, &s->agate, aq));
-    A_(salloc(s, &s->scores, (size_t)a.nh * s->kvcap));
-    {
-        const size_t nch = (size_t)oh_flash_slots(s->kvcap);
-        A_(salloc(s, &s->fpo, (size_t)a.nh * nch * a.hd + 64));
-        A_(salloc(s, &s->fpml, (size_t)a.nh * nch * 2 + 64));
-    }
-    A_(salloc(s, &s->ddots, (size_t)(K + 1) * H + 64));
-    A_(salloc(s, &s->dcnt, (size_t)H + 64));
-    A_(salloc(s, &s->osz, (size_t)a.nv * a.dv + 64));
-    A_(salloc(s, &s->oruns, (size_t)a.nv * a.dv / 16 + 64));
-    if (a.ne > 0) {
-        A_(salloc(s, &s->rtag, (size_t)a.n_layers * (a.ne + 1)));
-        A_(salloc(s, &s->mctr, (size_t)a.n_layers * 2));
-        A_(salloc(s, &s->dmctr, (size_t)a.n_layers * 2));
-    }
+    s->ls.resize((size_t)a.n_layers);
     {
         const char *e = getenv("ORNITH_HIP_EXACT_ATTN_MAX");
         if (e && *e) s->exact_max = s->pf_exact_max = atoi(e);
         const char *f = getenv("ORNITH_HIP_FLASH_MFMA");
         if (f && *f) s->flash_mfma = atoi(f) != 0;
     }
-    A_(salloc(s, &s->rl, a.ne > 0 ? a.ne : 1)); A_(salloc(s, &s->shl, 1)); A_(salloc(s, &s->shg, 1));
-    A_(salloc(s, &s->ew, 64)); A_(salloc(s, &s->eidx, 64));
-    const size_t nvec = (size_t)(K + 1);
-    A_(salloc(s, &s->g, nvec * I)); A_(salloc(s, &s->u, nvec * I)); A_(salloc(s, &s->h, nvec * I));
-    A_(q8alloc(s, s->hq, nvec * I));
-    A_(salloc(s, &s->od, nvec * H));
-    A_(salloc(s, &s->logits, a.vocab));
-    A_(salloc(s, &s->amv, OH_ARGMAX_BLOCKS)); A_(salloc(s, &s->ami, OH_ARGMAX_BLOCKS));
-    s->ls.resize((size_t)a.n_layers);
-    bool any_full = false;
-    for (int l = 0; l < a.n_layers; l++) {
-        LayerState &y = s->ls[l];
-        if (m->L[l].full) {
-            any_full = true;
-            A_(salloc(s, &y.Kt, (size_t)a.nkv * (a.hd / 4) * s->kvcap));
-            A_(salloc(s, &y.Ks, (size_t)s->kvcap * a.nkv));
-            A_(salloc(s, &y.Vq, (size_t)s->kvcap * a.nkv * a.hd));
-            A_(salloc(s, &y.Vh, (size_t)s->kvcap * a.nkv * a.hd));
-            A_(salloc(s, &y.Vs, (size_t)s->kvcap * a.nkv));
-        } else {
-            A_(salloc(s, &y.S, (size_t)a.nv * a.dk * a.dv));
-            A_(salloc(s, &y.conv, 2 * (size_t)(a.conv_k - 1) * cc));
+    auto lay = [&]() -> int {
+        CHK(salloc(s, &s->io, 64));
+        CHK(salloc(s, &s->toks, (size_t)cap + 1));
+        CHK(salloc(s, &s->x, H)); CHK(salloc(s, &s->xn, H)); CHK(q8alloc(s, s->xq, H));
+        CHK(salloc(s, &s->cat, cc > 0 ? cc : 1)); CHK(salloc(s, &s->gate, vd > 0 ? vd : 1));
+        CHK(salloc(s, &s->ab, 2 * (a.nv > 0 ? a.nv : 1)));
+        CHK(salloc(s, &s->o, ow)); CHK(q8alloc(s, s->oq, ow));
+        CHK(salloc(s, &s->qproj, 2 * (size_t)aq)); CHK(salloc(s, &s->kb, kvd)); CHK(salloc(s, &s->vb, kvd));
+        CHK(salloc(s, &s->qr, aq)); CHK(salloc(s, &s->agate, aq));
+        CHK(salloc(s, &s->scores, (size_t)a.nh * s->kvcap));
+        {
+            const size_t nch = (size_t)oh_flash_slots(s->kvcap);
+            CHK(salloc(s, &s->fpo, (size_t)a.nh * nch * a.hd + 64));
+            CHK(salloc(s, &s->fpml, (size_t)a.nh * nch * 2 + 64));
         }
-    }
-    if (any_full) {
-        // RoPE cos/sin per (pos, pair) with the reference's libm calls
-        // (ot_rope_partial, src/ornith_tensor.c:167-178)
-        int rot = a.rope_dim;
-        if (rot <= 0 || rot > a.hd) rot = a.hd;
-        const int half = a.hd / 2;
-        std::vector<float2> tab((size_t)cap * half);
-        std::vector<float> freq((size_t)rot / 2);
-        for (int i = 0; i < rot / 2; i++) freq[i] = powf(a.rope_theta, -2.0f * (float)i / (float)rot);
-        for (int p = 0; p < cap; p++)
-            for (int i = 0; i < half; i++) {
-                float2 cs = {1.0f, 0.0f};
-                if (i < rot / 2) {
-                    const float ang = (float)p * freq[i];
-                    cs.x = cosf(ang);
-                    cs.y = sinf(ang);
-                }
-                tab[(size_t)p * half + i] = cs;
+        CHK(salloc(s, &s->ddots, (size_t)(K + 1) * H + 64));
+        CHK(salloc(s, &s->dcnt, (size_t)H + 64));
+        CHK(salloc(s, &s->osz, (size_t)a.nv * a.dv + 64));
+        CHK(salloc(s, &s->oruns, (size_t)a.nv * a.dv / 16 + 64));
+        if (a.ne > 0) {
+            CHK(salloc(s, &s->rtag, (size_t)a.n_layers * (a.ne + 1)));
+            CHK(salloc(s, &s->mctr, (size_t)a.n_layers * 2));
+            CHK(salloc(s, &s->dmctr, (size_t)a.n_layers * 2));
+        }
+        CHK(salloc(s, &s->rl, a.ne > 0 ? a.ne : 1)); CHK(salloc(s, &s->shl, 1)); CHK(salloc(s, &s->shg, 1));
+        CHK(salloc(s, &s->ew, 64)); CHK(salloc(s, &s->eidx, 64));
+        const size_t nvec = (size_t)(K + 1);
+        CHK(salloc(s, &s->g, nvec * I)); CHK(salloc(s, &s->u, nvec * I)); CHK(salloc(s, &s->h, nvec * I));
+        CHK(q8alloc(s, s->hq, nvec * I));
+        CHK(salloc(s, &s->od, nvec * H));
+        CHK(salloc(s, &s->logits, a.vocab));
+        CHK(salloc(s, &s->amv, OH_ARGMAX_BLOCKS)); CHK(salloc(s, &s->ami, OH_ARGMAX_BLOCKS));
+        for (int l = 0; l < a.n_layers; l++) {
+            LayerState &y = s->ls[l];
+            if (m->L[l].full) {
+                CHK(salloc(s, &y.Kt, (size_t)a.nkv * (a.hd / 4) * s->kvcap));
+                CHK(salloc(s, &y.Ks, (size_t)s->kvcap * a.nkv));
+                CHK(salloc(s, &y.Vq, (size_t)s->kvcap * a.nkv * a.hd));
+                CHK(salloc(s, &y.Vh, (size_t)s->kvcap * a.nkv * a.hd));
+                CHK(salloc(s, &y.Vs, (size_t)s->kvcap * a.nkv));
+            } else {
+                CHK(salloc(s, &y.S, (size_t)a.nv * a.dk * a.dv));
+                CHK(salloc(s, &y.conv, 2 * (size_t)(a.conv_k - 1) * cc));
             }
-        A_(salloc(s, &s->rope, tab.size()));
-        hipError_t e = hipMemcpy(s->rope, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
-        if (e != hipSuccess) { ornith_hip_session_free(s); seterr("rope upload: %s", hipGetErrorString(e)); return ORNITH_HIP_ERR_DEVICE; }
-    }
+        }
+        return ORNITH_HIP_OK;
+    };
+    int st = slayout(s, lay);
+    if (st == ORNITH_HIP_OK && m->any_full) st = rope_table(m, s);
+    if (st != ORNITH_HIP_OK) { ornith_hip_session_free(s); return st; }
     // a session long enough for matrix-core prompt chunks has the model's
     // prompt tiles built here, once per model, outside its prompts
-    if (cap >= kMmqMinTokens) A_(pf_tiles(m, m->ctx->st));
-#undef A_
+    if (cap >= kMmqMinTokens && (st = pf_tiles(m, m->ctx->st)) != ORNITH_HIP_OK) {
+        ornith_hip_session_free(s);
+        return st;
+    }
     *out = s;
     return ORNITH_HIP_OK;
 }

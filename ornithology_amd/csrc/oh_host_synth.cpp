@@ -34,7 +34,7 @@ extern "C" int ornith_hip_model_synth(ornith_hip_ctx *ctx, const ornith_hip_gen_
     upd((uint64_t)H * cc); upd((uint64_t)H * 2 * c->nh * c->hd); upd((uint64_t)H * c->moe_inter * c->ne);
     upd((uint64_t)c->nh * c->hd * H); upd((uint64_t)vd * H); upd((uint64_t)H * c->shared_inter);
     float *tmp = nullptr;
-    HCHK(hipMalloc(&tmp, mx * 4 + 256));
+    HCHK(dev_malloc(ctx, (void **)&tmp, mx * 4 + 256));
     auto *m = new ornith_hip_model();
     m->ctx = ctx;
     hipStream_t st = ctx->st;
