@@ -190,33 +190,24 @@ extern "C" int ornith_hip_quantize(ornith_hip_ctx *ctx, uint32_t type, const flo
     if (n == 0 || n % 256) { seterr("quantize: %llu values is not a whole number of 256-blocks", (unsigned long long)n); return ORNITH_HIP_ERR_FORMAT; }
     HCHK(hipSetDevice(ctx->device));
     // the planes and the values in one block of the pool
-    ornith_hip_tensor t;
-    t.ctx = ctx;
-    t.name = "quantize";
-    t.type = type;
-    t.nd = 2;
-    t.dims[0] = 256;
-    t.dims[1] = n / 256;
-    t.in = 256;
-    t.rows = (int64_t)(n / 256);
-    t.gguf_bytes = gguf_nbytes(type, n);
     size_t pa, pb, pc;
-    plane_bytes(type, t.rows, t.in, &pa, &pb, &pc);
+    plane_bytes(type, (int64_t)(n / 256), 256, &pa, &pb, &pc);
     DevBlock blk;
     hipError_t e = dev_get(ctx, up256(pa) + up256(pb) + up256(pc) + n * 4, &blk);
     if (e != hipSuccess) { seterr("quantize: %s", hipGetErrorString(e)); return ORNITH_HIP_ERR_OOM; }
-    t.mem = t.A = (uint8_t *)blk.p;
-    t.B = t.A + up256(pa);
-    t.C = t.B + up256(pb);
-    float *dx = (float *)(t.C + up256(pc));
+    uint8_t *A = (uint8_t *)blk.p, *B = A + up256(pa), *C = B + up256(pb);
+    float *dx = (float *)(C + up256(pc));
     e = hipMemcpyAsync(dx, x, n * 4, hipMemcpyHostToDevice, ctx->st);
-    if (e == hipSuccess) e = oh_launch_encode(dx, (int)type, (int64_t)(n / 256), t.A, t.B, t.C, ctx->st);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->st);
-    int r = ORNITH_HIP_OK;
-    if (e != hipSuccess) { seterr("quantize: %s", hipGetErrorString(e)); r = ORNITH_HIP_ERR_DEVICE; }
-    if (r == ORNITH_HIP_OK) r = ornith_hip_tensor_download(&t, out, t.gguf_bytes);
+    if (e == hipSuccess) e = oh_launch_encode(dx, (int)type, (int64_t)(n / 256), A, B, C, ctx->st);
+    // the blocks in GGUF order over the values, which are used up
+    const int size = (int)gguf_nbytes(type, 256);
+    if (e == hipSuccess) e = oh_launch_gguf_pack(A, B, C, (int)type, size, 0, (int64_t)(n / 256), dx, ctx->st);
+    if (e == hipSuccess) e = hipMemcpyAsync(out, dx, n / 256 * (uint64_t)size, hipMemcpyDeviceToHost, ctx->st);
+    const hipError_t es = hipStreamSynchronize(ctx->st);
     dev_put(ctx, blk);
-    return r;
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) { seterr("quantize: %s", hipGetErrorString(e)); return ORNITH_HIP_ERR_DEVICE; }
+    return ORNITH_HIP_OK;
 }
 
 extern "C" int ornith_hip_dequant(ornith_hip_ctx *ctx, const ornith_hip_tensor *W,

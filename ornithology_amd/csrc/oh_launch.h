@@ -66,6 +66,10 @@ hipError_t oh_launch_mmq_tiles(const uint8_t *A, const uint8_t *B, uint8_t *PA, 
 hipError_t oh_launch_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32_t *list, int32_t *items,
                                 hipStream_t st);
 hipError_t oh_launch_iq2_slots(const oh_iq2rows *a, int max_items, hipStream_t st);
+// super-blocks [b0, b0 + n) of a quantised tensor's planes as GGUF blocks (size:
+// GGUF bytes of a super-block)
+hipError_t oh_launch_gguf_pack(const uint8_t *A, const uint8_t *B, const uint8_t *C, int type, int size, int64_t b0,
+                               int64_t n, void *out, hipStream_t st);
 // decode of n sessions at once: the decode bodies, one grid row per session,
 // descriptors and positions in device arrays of n
 hipError_t oh_launch_delta_batch(const oh_op_delta *ops, const int32_t *pos, int n, int dk, int K, int nv,
