@@ -22,6 +22,7 @@
 // weights is being fetched.
 #include "oh_common.h"
 #include "oh_types.h"
+#include "oh_dpp.h"
 #include "oh_iq2.h"
 
 namespace {
@@ -431,14 +432,47 @@ OH_HD inline int mv_lds_iq2t_off(int nb, int in) { return mv_lds_iq2_off(nb, in)
 // the split form's scales d: [OH_IQ2_ROWS][nb] halves after the two term tiles
 OH_HD inline int mv_lds_iq2d_off(int nb, int in) { return mv_lds_iq2t_off(nb, in) + 2 * OH_IQ2_ROWS * kIq2S * 4; }
 
-// Eight terms of one codebook entry: (db * +-g_j) * x_j, the grid bytes of
-// entry gv carrying their signs (sm: the entry's sign masks); (db * -g) * x
-// is -((db * g) * x) exactly.
-OH_DEV void iq2_terms8(uint64_t gv, const uint4 sm, float db, const float4 x0, const float4 x1, float (&ts)[8]) {
-    const uint32_t gs[2] = {((uint32_t)gv ^ sm.x) + sm.z, ((uint32_t)(gv >> 32) ^ sm.y) + sm.w};
-    const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+// A sub-block's four codebook entries with their signs: byte j of word 2 k + h
+// is +-g of element 8 k + 4 h + j.
+struct Iq2Look { uint64_t g[4]; uint4 m[4]; };
+OH_DEV Iq2Look iq2_look(const uint64_t *grid, const uint4 *stab, uint32_t w0, uint32_t w1) {
+    Iq2Look l;
 #pragma unroll
-    for (int j = 0; j < 8; j++) ts[j] = db * (float)(int8_t)(gs[j / 4] >> (8 * (j % 4))) * xs[j];
+    for (int k = 0; k < 4; k++) {
+        l.g[k] = grid[(w0 >> (8 * k)) & 0xffu];
+        l.m[k] = stab[(w1 >> (7 * k)) & 127u];
+    }
+    return l;
+}
+// The sub-block's 32 terms (db * +-g) * x in element order, four at a time:
+// use(k, t) takes the terms of elements 4 k .. 4 k + 3. x: two elements per lane
+// of each 16-lane row, entering the products as DPP broadcasts; (db * -g) * x
+// is -((db * g) * x) exactly. The next four weights are formed between the
+// products and their use.
+template <class F>
+OH_DEV void iq2_terms(const Iq2Look &l, float db, const float2 x, F &&use) {
+    auto weights = [&](int k, float (&w)[4]) {
+        const uint32_t g = k & 1 ? (uint32_t)(l.g[k >> 1] >> 32) : (uint32_t)l.g[k >> 1];
+        const uint4 m = l.m[k >> 1];
+        const uint32_t gs = (g ^ (k & 1 ? m.y : m.x)) + (k & 1 ? m.w : m.z);
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = db * (float)(int8_t)(gs >> (8 * j));
+    };
+    float w[4];
+    weights(0, w);
+    static_for<8>([&](auto k_) {
+        constexpr int k = k_;
+        float t[4];
+        order();
+        static_for<4>([&](auto j_) {
+            constexpr int j = j_;
+            t[j] = row_lane<2 * k + j / 2>(j % 2 ? x.y : x.x) * w[j];
+        });
+        order();
+        if constexpr (k < 7) weights(k + 1, w);
+        order();
+        use(k_, t);
+    });
 }
 
 OH_DEV void iq2_rows_lane(const oh_mvseg &s, int slot, int blk, int expert, uint8_t *smem) {
@@ -466,22 +500,25 @@ OH_DEV void iq2_rows_lane(const oh_mvseg &s, int slot, int blk, int expert, uint
     iq2_sign_table(stab);
     lds_barrier();
     float acc = 0.0f;
-    // super-block b: each term added at once, in element order
+    // super-block b: each term added at once, in element order; a sub-block's
+    // table entries are read while the one before it is added
+    const float2 *xl = (const float2 *)v + (tid & 15);
     auto reduce = [&](int b, const uint4 (&q)[4], uint32_t d) {
         const float dd = h2f((uint16_t)d);
-        const float4 *xb = (const float4 *)(v + b * 256);
+        float2 x[8];
+#pragma unroll
+        for (int g32 = 0; g32 < 8; g32++) x[g32] = xl[b * 128 + g32 * 16];
+        Iq2Look l = iq2_look(grid, stab, q[0].x, q[0].y);
 #pragma unroll
         for (int g32 = 0; g32 < 8; g32++) {
-            const uint32_t w0 = wsel(q[g32 >> 1], 2 * (g32 & 1)), w1 = wsel(q[g32 >> 1], 2 * (g32 & 1) + 1);
-            const float db = dd * (0.5f + (float)(w1 >> 28)) * 0.25f;
+            const float db = dd * (0.5f + (float)(wsel(q[g32 >> 1], 2 * (g32 & 1) + 1) >> 28)) * 0.25f;
+            const Iq2Look cur = l;
+            if (g32 < 7) l = iq2_look(grid, stab, wsel(q[(g32 + 1) >> 1], 2 * ((g32 + 1) & 1)),
+                                      wsel(q[(g32 + 1) >> 1], 2 * ((g32 + 1) & 1) + 1));
+            iq2_terms(cur, db, x[g32], [&](auto, const float (&t)[4]) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                float ts[8];
-                iq2_terms8(grid[(w0 >> (8 * k)) & 0xffu], stab[(w1 >> (7 * k)) & 127u], db,
-                           xb[g32 * 8 + 2 * k], xb[g32 * 8 + 2 * k + 1], ts);
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc += ts[j];
-            }
+                for (int j = 0; j < 4; j++) acc += t[j];
+            });
         }
     };
     int b = 0;
@@ -558,16 +595,11 @@ OH_DEV void iq2_rows(const oh_mvseg &s, int slot, int blk, int expert, uint8_t *
             if (sb < nsb) {
                 const float dd = h2f(dh[sb / 8]);
                 const float db = dd * (0.5f + (float)(w1 >> 28)) * 0.25f;
-                const float4 *xb = (const float4 *)(v + sb * 32);
+                const float2 x = *((const float2 *)(v + sb * 32) + (lane & 15));
                 float *dst = tile + ((c & 1) * OH_IQ2_ROWS + lane) * kIq2S + (wave - 1) * 32;
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    float ts[8];
-                    iq2_terms8(grid[(w0 >> (8 * k)) & 0xffu], stab[(w1 >> (7 * k)) & 127u], db, xb[2 * k],
-                               xb[2 * k + 1], ts);
-                    *(float4 *)(dst + 8 * k) = make_float4(ts[0], ts[1], ts[2], ts[3]);
-                    *(float4 *)(dst + 8 * k + 4) = make_float4(ts[4], ts[5], ts[6], ts[7]);
-                }
+                iq2_terms(iq2_look(grid, stab, w0, w1), db, x, [&](auto k, const float (&t)[4]) {
+                    *(float4 *)(dst + 4 * decltype(k)::value) = make_float4(t[0], t[1], t[2], t[3]);
+                });
             }
         }
         if (wave == 0 && c > 0) {
