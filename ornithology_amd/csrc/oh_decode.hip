@@ -783,7 +783,6 @@ OH_DEV void dop_prep(const oh_datt &d, int vb, const Dctl &c) {
             } else {
                 const size_t vo = (((size_t)h * (cap / 16) + pos / 16) * hd + t) * 16 + (pos & 15);
                 if (t < hd) stc(a.Vq + vo, (int8_t)code);
-                if (t < hd && a.Vh) stc(a.Vh + vo, f16_bits_of_code(code));
                 if (t == 0) stc(a.Vs + off, scale);
             }
         }

@@ -178,7 +178,6 @@ struct LayerState {
     float *S = nullptr, *conv = nullptr;                 // linear
     uint32_t *Kt = nullptr; float *Ks = nullptr;         // full (Q8 KV)
     int8_t *Vq = nullptr; float *Vs = nullptr;
-    uint16_t *Vh = nullptr;       // the V codes as f16 bits in the same tiles (the exact walk's operand)
 };
 
 struct ornith_hip_session {

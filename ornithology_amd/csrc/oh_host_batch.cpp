@@ -97,7 +97,6 @@ std::string batch_check(ornith_hip_session *const *ss, int n, const std::vector<
                 BC(sb, pr.Kt, kvd / 4 * cap * 4, "K codes");
                 BC(sb, pr.Ks, cap * a.nkv * F, "K scales");
                 BC(sb, pr.Vq, cap * kvd, "V codes");
-                BC(sb, pr.Vh, cap * kvd * 2, "V codes (f16)");
                 BC(sb, pr.Vs, cap * a.nkv * F, "V scales");
                 if (at.qr != pr.qr || at.gate != pr.gate || at.Kt != pr.Kt || at.Ks != pr.Ks || at.Vq != pr.Vq ||
                     at.Vs != pr.Vs) {
@@ -414,7 +413,7 @@ static int batch_step_off(ornith_hip_session **ss, int n, const int32_t *tokens,
                 oh_op_prep pr = {p.QP + (size_t)b * 2 * aq, p.KB + (size_t)b * kvd, p.VB + (size_t)b * kvd,
                                  (const float *)y.q_norm->A, (const float *)y.k_norm->A, (const float *)sb->rope,
                                  p.QR + (size_t)b * aq, p.AG + (size_t)b * aq, z.Kt, z.Ks, z.Vq, z.Vs,
-                                 a.nh, a.nkv, a.hd, a.rope_dim, sb->kvcap, a.eps, z.Vh};
+                                 a.nh, a.nkv, a.hd, a.rope_dim, sb->kvcap, a.eps};
                 memcpy(dst + (size_t)b * sizeof(oh_op_prep), &pr, sizeof pr);
                 oh_op_attn at;
                 memset(&at, 0, sizeof at);

@@ -196,7 +196,6 @@ extern "C" int ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_s
                 CHK(salloc(s, &y.Kt, (size_t)a.nkv * (a.hd / 4) * s->kvcap));
                 CHK(salloc(s, &y.Ks, (size_t)s->kvcap * a.nkv));
                 CHK(salloc(s, &y.Vq, (size_t)s->kvcap * a.nkv * a.hd));
-                CHK(salloc(s, &y.Vh, (size_t)s->kvcap * a.nkv * a.hd));
                 CHK(salloc(s, &y.Vs, (size_t)s->kvcap * a.nkv));
             } else {
                 CHK(salloc(s, &y.S, (size_t)a.nv * a.dk * a.dv));
@@ -247,7 +246,7 @@ int build_body(ornith_hip_session *s, Prog &P) {
                 oh_op o = op_new(OH_OP_ATTN_PREP, a.nh + a.nkv);
                 o.u.prep = {s->qproj, s->kb, s->vb, (const float *)y.q_norm->A, (const float *)y.k_norm->A,
                             (const float *)s->rope, s->qr, s->agate, z.Kt, z.Ks, z.Vq, z.Vs,
-                            a.nh, a.nkv, a.hd, a.rope_dim, s->kvcap, a.eps, z.Vh};
+                            a.nh, a.nkv, a.hd, a.rope_dim, s->kvcap, a.eps};
                 prog_add(P, o, K_ATTN_PREP, 4.0 * (2.0 * aqd + 2.0 * kvd + 2.0 * a.hd) + 8.0 * aqd +
                                                 2.0 * (kvd + 4.0 * a.nkv));
             }
@@ -257,7 +256,7 @@ int build_body(ornith_hip_session *s, Prog &P) {
             const bool ex = s->qpos + 1 <= oh_exact_limit(s->exact_max, a.hd);
             oh_op_attn at;
             memset(&at, 0, sizeof at);
-            at.qr = s->qr; at.gate = s->agate; at.Kt = z.Kt; at.Ks = z.Ks; at.Vq = z.Vq; at.Vs = z.Vs; at.Vh = z.Vh;
+            at.qr = s->qr; at.gate = s->agate; at.Kt = z.Kt; at.Ks = z.Ks; at.Vq = z.Vq; at.Vs = z.Vs;
             at.scores = s->scores; at.part_o = s->fpo; at.part_ml = s->fpml; at.out = s->o;
             at.nh = a.nh; at.nkv = a.nkv; at.hd = a.hd; at.cap = s->kvcap; at.exact_max = s->exact_max;
             at.hb = oh_flash_form(a.nh, a.nkv, a.hd, s->flash_mfma); at.scale = scale;
@@ -271,15 +270,14 @@ int build_body(ornith_hip_session *s, Prog &P) {
                 // graph step, exact regime (the host picks this program
                 // while the context fits the exact walk): the scores over
                 // 64-position tiles of every KV head, then one block per
-                // query head for the softmax and the output walk
+                // 64 dimensions of a query head for the softmax and the output walk
                 const int lim = oh_exact_limit(s->exact_max, a.hd);
                 oh_op o3 = op_new(OH_OP_ATTN_SCORES, a.nkv * ((lim + 63) / 64), ((a.nh / a.nkv) * 4 + 64) * a.hd);
                 o3.u.attn = at;
                 prog_add(P, o3, K_ATTN_SCORES, kvb + 4.0 * T * a.nh + 4.0 * aqd);
-                oh_op o4 = op_new(OH_OP_ATTN_WALK, a.nh, ((lim + 15) / 16 + 2) * 16 * 4);
+                oh_op o4 = op_new(OH_OP_ATTN_WALK, oh_attn_walk_blocks(a.nh, a.hd), oh_attn_walk_lds(lim));
                 o4.u.attn = at;
-                // the walk reads the f16 copy of the codes (2 bytes each) and the scales
-                prog_add(P, o4, K_ATTN_WALK, T * a.nkv * (2.0 * a.hd + 4.0) + 4.0 * T * a.nh + 12.0 * aqd);
+                prog_add(P, o4, K_ATTN_WALK, T * a.nkv * (a.hd + 4.0) + 4.0 * T * a.nh + 12.0 * aqd);
             } else {
                 const int nv_ex = a.nh / (256 / a.hd), lds_ex = oh_exact_lds_bytes(a.hd, s->exact_max);
                 oh_op o3 = op_new(OH_OP_ATTN_MAIN, nv_ex > nv_fl ? nv_ex : nv_fl, lds_ex > lds_fl ? lds_ex : lds_fl);
@@ -776,7 +774,7 @@ bool dec_build(ornith_hip_session *s, DecB &b) {
             o.nvb = a.nh + a.nkv;
             o.u.at.p = {nullptr, nullptr, nullptr, (const float *)y.q_norm->A, (const float *)y.k_norm->A,
                         (const float *)s->rope, s->qr, s->agate, z.Kt, z.Ks, z.Vq, z.Vs,
-                        a.nh, a.nkv, a.hd, a.rope_dim, s->kvcap, a.eps, z.Vh};
+                        a.nh, a.nkv, a.hd, a.rope_dim, s->kvcap, a.eps};
             o.u.at.qkv = qkv;
             o.u.at.flags = pflags;
             b.ops.push_back(o);

@@ -70,6 +70,10 @@ hipError_t oh_launch_iq2_slots(const oh_iq2rows *a, int max_items, hipStream_t s
 // GGUF bytes of a super-block)
 hipError_t oh_launch_gguf_pack(const uint8_t *A, const uint8_t *B, const uint8_t *C, int type, int size, int64_t b0,
                                int64_t n, void *out, hipStream_t st);
+// the exact walk's launch: blocks and dynamic LDS for contexts up to lim
+int oh_attn_walk_blocks(int nh, int hd);
+int oh_attn_walk_lds(int lim);
+hipError_t oh_launch_attn_walk(const oh_op_attn *a, const int32_t *io, int blocks, int lds_bytes, hipStream_t st);
 // decode of n sessions at once: the decode bodies, one grid row per session,
 // descriptors and positions in device arrays of n
 hipError_t oh_launch_delta_batch(const oh_op_delta *ops, const int32_t *pos, int n, int dk, int K, int nv,

@@ -34,14 +34,6 @@ OH_DEV uint32_t bsel(const uint4 &v, int k) {   // byte k of a uint4
     return (wsel(v, k >> 2) >> (8 * (k & 3))) & 0xffu;
 }
 
-// Block barrier that orders LDS only: it does not wait for the block's
-// outstanding global loads (prefetched weights).
-OH_DEV void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // 6-bit (scale, min) of sub-block j from the 12 packed bytes that start at
 // byte 4 of the Q4_K header (src/ornith_qdot.c:66-72).
 OH_DEV void q4k_sm(const uint4 &hdr, int j, int &sc, int &mn) {

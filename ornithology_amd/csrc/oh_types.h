@@ -250,7 +250,6 @@ typedef struct {
     float *Vs;
     int nh, nkv, hd, rot, cap;
     float eps;
-    uint16_t *Vh;                  // the V codes again as f16 bits, same tiles (optional)
 } oh_op_prep;
 
 // GQA scores / ordered output / flash chunks / flash merge
@@ -263,7 +262,6 @@ typedef struct {
     float *scores, *part_o, *part_ml, *out;
     int nh, nkv, hd, cap, exact_max, hb;
     float scale;
-    const uint16_t *Vh;            // the V codes as f16 bits (the graph step's exact walk)
 } oh_op_attn;
 
 typedef struct {
@@ -322,6 +320,19 @@ typedef struct {
     const int32_t *off, *list, *items;
     int in, rows, xstride, ystride, adiv, cols;
 } oh_iq2rows;
+
+// Longest context of the decode step's exact walk for head dim hd: the
+// scores of the block's 256/hd heads stay in LDS, at most 48 KB of it
+// (8192 positions at hd 256, 6144 at 128, 3072 at 64).
+OH_HD static inline int exact_cap(int hd) {
+    const int c = 12288 * hd / 256;
+    return c < 8192 ? c : 8192;
+}
+// the decode step's exact-walk limit for a session's exact_max
+OH_HD static inline int exact_lim(int exact_max, int hd) {
+    const int c = exact_cap(hd);
+    return exact_max < c ? (exact_max > 0 ? exact_max : 0) : c;
+}
 
 // Persistent step kernel: counters of one program phase (one per 64-byte
 // line, OH_STEP_NCTR of them) and the io words it uses.
