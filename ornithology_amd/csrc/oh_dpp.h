@@ -26,3 +26,12 @@ OH_DEV int again(int i) { asm volatile("" : "+v"(i)); return i; }
 // one that it only overwrites, so products and sums are kept in groups: left
 // to itself the compiler pairs each product with its sum and a wait.
 OH_DEV void order() { __builtin_amdgcn_sched_barrier(0); }
+// lane l + I of the 16-lane row, in lane l; opaque, so that a chain of adds over
+// several of them is plain adds: folded into its add's DPP operand each would
+// wait two slots for the running sum that the add before it wrote
+template <int I>
+OH_DEV float row_ahead(float v) {
+    float u = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x100 + I, 0xf, 0xf, true));
+    asm volatile("" : "+v"(u));
+    return u;
+}

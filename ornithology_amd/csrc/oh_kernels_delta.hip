@@ -347,7 +347,7 @@ oh_k_delta_chunked(const float *qn, const float *kn, const float *conv, const fl
                     chain<i>(
                         [&](auto k_) {
                             constexpr int j = i - 1 - k_;
-                            return row_lane<(j & 15)>(j < 16 ? f4(ml[i / 4], i & 3) : f4(mh[i / 4 - (j < 16 ? 0 : C / 8)], i & 3)) * u[j];
+                            return row_lane<(j & 15)>(j < 16 ? f4(ml[i / 4], i & 3) : f4(mh[i / 4 % (C / 8)], i & 3)) * u[j];
                         },
                         [&](auto, float t) { u[i] = u[i] - t; });
                 });
@@ -357,7 +357,7 @@ oh_k_delta_chunked(const float *qn, const float *kn, const float *conv, const fl
                     float ui = u[i];
                     static_for<i>([&](auto j_) {
                         constexpr int j = i - 1 - j_;
-                        const float m = row_lane<(j & 15)>(j < 16 ? f4(ml[i / 4], i & 3) : f4(mh[i / 4 - (j < 16 ? 0 : C / 8)], i & 3));
+                        const float m = row_lane<(j & 15)>(j < 16 ? f4(ml[i / 4], i & 3) : f4(mh[i / 4 % (C / 8)], i & 3));
                         const float t = m != 0.0f ? m * u[j] : 0.0f;
                         ui = ui - t;
                     });

@@ -46,6 +46,55 @@ OH_DEV void q4k_sm(const uint4 &hdr, int j, int &sc, int &mn) {
     }
 }
 
+// The nb terms of a row, in lanes base .. base + nb - 1, added in order from 0;
+// the result is the row's only in lane base. A cross-lane read per add made
+// this a chain of LDS round trips, about 0.4 us of every matrix-vector launch
+// at 8 super-blocks (a 4096-position decode step of 40 layers: 2715 -> 2618 us
+// with squares() below): where a row stays within 16 lanes (a power of two of them, so
+// base is a multiple of it) its terms come by DPP and only the adds are serial;
+// otherwise eight reads travel together.
+template <int N>
+OH_DEV float row_terms16(float t) {
+    float u[N];
+    static_for<N - 1>([&](auto i_) { constexpr int i = i_; u[i + 1] = row_ahead<i + 1>(t); });
+    float acc = 0.0f + t;
+#pragma unroll
+    for (int i = 1; i < N; i++) acc += u[i];
+    return acc;
+}
+OH_DEV float row_terms(float t, int base, int nb) {
+    switch (nb) {
+    case 2: return row_terms16<2>(t);
+    case 4: return row_terms16<4>(t);
+    case 8: return row_terms16<8>(t);
+    case 16: return row_terms16<16>(t);
+    }
+    float acc = 0.0f;
+    for (int i0 = 0; i0 < nb; i0 += 8) {
+        float u[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) u[i] = shfl(t, base + i0 + i);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (i0 + i < nb) acc += u[i];
+    }
+    return acc;
+}
+// A thread's part of sum v[i]^2, i = tid, tid + 256, .. in that order; eight
+// reads travel together.
+OH_DEV double squares(const float *v, int n, int tid) {
+    double ss = 0.0;
+    for (int i0 = tid; i0 < n; i0 += 2048) {
+        float q[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = v[i0 + 256 * k < n ? i0 + 256 * k : tid];
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            if (i0 + 256 * k < n) ss += (double)q[k] * q[k];
+    }
+    return ss;
+}
+
 OH_DEV int group_isum(int v) {     // exact sum over the 8 lanes of a group
     v += shfl_xor(v, 1); v += shfl_xor(v, 2); v += shfl_xor(v, 4);
     return v;
@@ -767,9 +816,7 @@ OH_DEV void mv_prologue(const oh_mvseg &s, int slot, int blk, uint8_t *smem, dou
             // the weights are requested before the reduction; the sum of
             // squares in the order of the stand-alone RMSNorm kernel
             const float4 *w4 = (const float4 *)s.nw;
-            double ss = 0.0;
-            for (int i = tid; i < in; i += 256) ss += (double)v[i] * v[i];
-            ss = wave_sum_d(ss);
+            const double ss = wave_sum_d(squares(v, in, tid));
             if (lane_id() == 0) red[wave] = ss;
             lds_barrier();
             const double tot = (red[0] + red[1]) + (red[2] + red[3]);
@@ -957,9 +1004,7 @@ OH_DEV void pro_compute(const PIn &p, const oh_mvseg &s, int slot, int blk, uint
         for (int k = 0; k < 4; k++)
             if (tid + 256 * k < n4) v4[tid + 256 * k] = fv[k];
         lds_barrier();
-        double ss = 0.0;
-        for (int i = tid; i < in; i += 256) ss += (double)v[i] * v[i];
-        ss = wave_sum_d(ss);
+        const double ss = wave_sum_d(squares(v, in, tid));
         if (lane_id() == 0) red[wave] = ss;
         lds_barrier();
         const double tot = (red[0] + red[1]) + (red[2] + red[3]);
@@ -1046,8 +1091,7 @@ OH_DEV void mv_seg(const oh_mvseg &s, int slot, int blk, int expert, uint8_t *sm
         const float tw = sb_term(r, aq, abs, *adp);
         const float t = live ? tw : 0.0f;
         // the row's super-block terms in order, from 0 (lanes rl*nb .. +nb-1)
-        float acc = 0.0f;
-        for (int i = 0; i < nb; i++) acc += shfl(t, rl * nb + i);
+        const float acc = row_terms(t, rl * nb, nb);
         if (s.pair) {
             if ((st & 1) == 0) gsum = acc;
             else if (live && sb == 0) emit<W::kGrid>(y, 0, row, ref_silu(gsum) * acc);
@@ -1704,8 +1748,7 @@ OH_DEV void down_body(const oh_mvdown &D, int vb, W &wt) {
                                      ((const float *)(b + mv_lds_d_off(nb)))[sb]);
             const bool live = rl < rps && row < D.rows;
             const float t = live ? tw : 0.0f;
-            float acc = 0.0f;
-            for (int i = 0; i < nb; i++) acc += shfl(t, rl * nb + i);
+            const float acc = row_terms(t, rl * nb, nb);
             if (rl < rps && sb == 0) dots[j * rps + rl] = acc;
         }
     }
@@ -1793,9 +1836,7 @@ OH_DEV void down_narrow(const oh_mvdown &D, int vb) {
                                  ((const float *)(b + mv_lds_d_off(nb)))[sb]);
         const bool live = act && row < D.rows;
         const float t = live ? tw : 0.0f;
-        const int base = lane - sb;
-        float acc = 0.0f;
-        for (int i = 0; i < nb; i++) acc += shfl(t, base + i);
+        const float acc = row_terms(t, lane - sb, nb);
         if (act && sb == 0) dots[j * R + rl] = acc;
     }
     lds_barrier();
@@ -1865,8 +1906,7 @@ OH_DEV void down_split(const oh_mvdown &D, int vb, W &wt) {
                              ((const float *)(q + mv_lds_d_off(nb)))[sb]);
     const bool live = act && rl < rps && row < D.rows;
     const float t = live ? tw : 0.0f;
-    float acc = 0.0f;
-    for (int i = 0; i < nb; i++) acc += shfl(t, rl * nb + i);
+    const float acc = row_terms(t, rl * nb, nb);
     if (live && sb == 0) stc(D.dots + (size_t)j * D.rows + row, acc);
     // count the block in its row group once every wave's stores completed
     __builtin_amdgcn_s_waitcnt(0);
@@ -1955,14 +1995,11 @@ OH_DEV void mvb_body(const oh_mvbatch &B) {
             const int16_t *abs = (const int16_t *)(cb + mv_lds_bs_off(nb)) + sb * 16;
             const float yd = ((const float *)(cb + mv_lds_d_off(nb)))[sb];
             const float t1 = rlive ? sb_term(r, aq, abs, yd) : 0.0f;
-            float acc = 0.0f;
-            for (int i = 0; i < nb; i++) acc += shfl(t1, rl * nb + i);
+            const float acc = row_terms(t1, rl * nb, nb);
             float out = acc;
             if (B.pair) {
                 const float t2 = rlive ? sb_term(r2, aq, abs, yd) : 0.0f;
-                float acc2 = 0.0f;
-                for (int i = 0; i < nb; i++) acc2 += shfl(t2, rl * nb + i);
-                out = ref_silu(acc) * acc2;
+                out = ref_silu(acc) * row_terms(t2, rl * nb, nb);
             }
             if (rlive && sb == 0) {
                 float *yp = B.y + (size_t)scol[c] * B.ystride + row;
@@ -2046,9 +2083,7 @@ oh_k_rmsnorm_q8k(const float *x, const float *norm_w, float eps, int n,
     for (int i = tid; i < n; i += 256) v[i] = x[i];
     __syncthreads();
     if (norm_w) {
-        double ss = 0.0;
-        for (int i = tid; i < n; i += 256) ss += (double)v[i] * v[i];
-        ss = wave_sum_d(ss);
+        const double ss = wave_sum_d(squares(v, n, tid));
         if (lane_id() == 0) red[wave] = ss;
         __syncthreads();
         const double tot = (red[0] + red[1]) + (red[2] + red[3]);
@@ -2168,9 +2203,7 @@ oh_k_norm_q8k_rows(const float *x, const float *norm_w, float eps, int n, float 
     }
     __syncthreads();
     if (norm_w) {
-        double ss = 0.0;
-        for (int i = tid; i < n; i += 256) ss += (double)v[i] * v[i];
-        ss = wave_sum_d(ss);
+        const double ss = wave_sum_d(squares(v, n, tid));
         if (lane_id() == 0) red[wave] = ss;
         __syncthreads();
         const double tot = (red[0] + red[1]) + (red[2] + red[3]);
