@@ -328,7 +328,8 @@ int pf_chunk(ornith_hip_session *s, int base, int T, bool chunked, hipStream_t s
                                 y.up_exps->rows == y.gate_exps->rows && y.up_exps->in == y.gate_exps->in;
                 const bool dn = (gu || pairable(y.gate_exps, y.up_exps)) && pf_iq2_slots(y.down_exps, T * K);
                 const int cols = pf_iq2_cols(T * K), slot_items = pf_iq2_items(T * K, a.ne);
-                if (gu || dn) HCHK(oh_launch_slot_lists(p.RIDX, T * K, a.ne, cols, p.CNT, p.LIST, p.ITEMS, st));
+                if (gu || dn) HCHK(oh_launch_slot_lists(p.RIDX, T * K, a.ne, cols, p.CNT, p.LIST, p.ITEMS,
+                                                            s->io + OH_IO_ERR, st));
                 Act ah;
                 ah.pro = OH_PRO_F32;
                 ah.xf = p.Hh;

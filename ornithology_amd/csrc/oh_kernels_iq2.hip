@@ -161,14 +161,20 @@ OH_DEV int block_incl_sum(int v, int32_t *sum) {
 // e's entries of list (their order does not matter: every slot is computed on
 // its own), items[0] the number of pieces of up to cols slots of one
 // expert, then (piece << 10 | expert) of each. One block; an expert picked
-// twice by one token keeps both entries.
+// twice by one token keeps both entries; an index outside [0, ne) is reported
+// and left out.
 __global__ void __launch_bounds__(kListThreads)
-oh_k_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32_t *list, int32_t *items) {
+oh_k_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32_t *list, int32_t *items,
+                int32_t *err) {
     __shared__ int32_t cnt[kListThreads], sum[kListThreads];
     const int tid = tid_x();
     cnt[tid] = 0;
     __syncthreads();
-    for (int p = tid; p < n; p += kListThreads) atomicAdd(&cnt[ldg(idx + p)], 1);
+    for (int p = tid; p < n; p += kListThreads) {
+        const int e = ldg(idx + p);
+        if (e >= 0 && e < ne) atomicAdd(&cnt[e], 1);
+        else atomicOr(err, OH_ERR_EXPERT_LIST);
+    }
     __syncthreads();
     const int mine = cnt[tid], np = (mine + cols - 1) / cols;
     const int end = block_incl_sum(mine, sum), pend = block_incl_sum(np, sum);
@@ -180,7 +186,10 @@ oh_k_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32
     }
     for (int k = 0; k < np; k++) stg(items + 1 + pend - np + k, (int32_t)(k << 10 | tid));
     __syncthreads();
-    for (int p = tid; p < n; p += kListThreads) stg(list + atomicAdd(&cnt[ldg(idx + p)], 1), (int32_t)p);
+    for (int p = tid; p < n; p += kListThreads) {
+        const int e = ldg(idx + p);
+        if (e >= 0 && e < ne) stg(list + atomicAdd(&cnt[e], 1), (int32_t)p);
+    }
 }
 
 } // namespace
@@ -188,9 +197,9 @@ oh_k_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32
 extern "C" {
 
 hipError_t oh_launch_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32_t *list, int32_t *items,
-                                hipStream_t st) {
+                                int32_t *err, hipStream_t st) {
     if (ne < 1 || ne > kListThreads || cols < 1 || cols > 8) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(oh_k_slot_lists, dim3(1), dim3(kListThreads), 0, st, idx, n, ne, cols, off, list, items);
+    hipLaunchKernelGGL(oh_k_slot_lists, dim3(1), dim3(kListThreads), 0, st, idx, n, ne, cols, off, list, items, err);
     return hipGetLastError();
 }
 

@@ -60,11 +60,11 @@ bool oh_mmq_can(uint32_t type, int rows, int in);
 hipError_t oh_launch_mmq_tiles(const uint8_t *A, const uint8_t *B, uint8_t *PA, uint8_t *PB, int64_t rows,
                                int nb, int P, hipStream_t st);
 // a chunk's IQ2_XXS experts: the slots grouped by expert (ne <= 1024; off: ne + 1
-// entries, list: n, items: those of up to cols (<= 8) slots each,
-// after their count), then
-// the rows of every expert over its slots
+// entries, list: n, items: those of up to cols (<= 8) slots each, after their
+// count; an index outside [0, ne) sets OH_ERR_EXPERT_LIST in *err and is left
+// out), then the rows of every expert over its slots
 hipError_t oh_launch_slot_lists(const int32_t *idx, int n, int ne, int cols, int32_t *off, int32_t *list, int32_t *items,
-                                hipStream_t st);
+                                int32_t *err, hipStream_t st);
 hipError_t oh_launch_iq2_slots(const oh_iq2rows *a, int max_items, hipStream_t st);
 // super-blocks [b0, b0 + n) of a quantised tensor's planes as GGUF blocks (size:
 // GGUF bytes of a super-block)
