@@ -66,19 +66,36 @@ bool pf_moe_slots_ok(const OhLayer &y) {
     return true;
 }
 
-// IQ2_XXS experts of at least this many (token, expert) slots run grouped by
-// expert, the weights formed once for up to cols slots; fewer slots keep the
-// token step's rows (a launch per slot and row, shorter chains). 512 experts,
-// top 10, gate/up 4096 -> 1024, one layer, a whole request in us, rows per slot
-// against groups of 4 and of 8: 400 slots 2038 / 2017 / 2263, 1280: 4604 / 4242 /
-// 4417, 2000: 7077 / 6169 / 6028, 5000: 15692 / 11513 / 10802
-constexpr int kIq2MinSlots = 480;
-bool pf_iq2_slots(const ornith_hip_tensor *W, int slots) {
-    return W->type == OH_IQ2_XXS && !iq2_tree_on() && slots >= kIq2MinSlots;
+// IQ2_XXS experts run grouped by expert, the weights formed once for up to cols
+// slots, from 480 (token, expert) slots; fewer keep the token step's rows (a
+// launch per slot and row, shorter chains). What decides is how much work there
+// is, more than how many slots share an expert: one layer, a prompt in us, rows
+// per slot against groups of 4,
+//   512 experts, 4096 -> 1024: 400 slots 2038 / 2017, 480: 1372 / 1233 (a later build)
+//   16 experts, 4096 -> 1024:  240: 1067 / 1068, 480: 1273 / 961
+//   512 experts, 4096 -> 512:  400: 731 / 761, 480: 806 / 793
+//   8, 32, 128, 256 experts, 2048 -> 512, at 480: 631 / 547, 597 / 587, 540 / 531, 524 / 524.
+// Where there are more experts than slots, of at most 2^20 weights a projection,
+// few weights are shared and groups gain nothing until they fill the chip: 1024
+// experts, 2048 -> 512: 560 slots 615 / 668, 720: 706 / 701, 800: 740 / 710; 768:
+// 560: 631 / 683; 1024, 2048 -> 256: 640: 499 / 546, 800: 562 / 567. (With 512 of
+// 2048 -> 512 it depends on the router: 560 slots 606 / 661 and 593 / 572.)
+constexpr int kIq2MinSlots = 480, kIq2MinThin = 760;
+bool pf_iq2_slots(const ornith_hip_tensor *W, int slots, int ne) {
+    if (W->type != OH_IQ2_XXS || iq2_tree_on()) return false;
+    const bool thin = (int64_t)W->rows * W->in <= (int64_t)ne << 20 && slots < ne;
+    return slots >= (thin ? kIq2MinThin : kIq2MinSlots);
 }
-int pf_iq2_cols(int n) { return n < 1800 ? 4 : 8; }
+// Groups of 8 need experts that fill them (the columns of a piece that only
+// repeat one are work for nothing), or so many slots that this is a small part.
+// Groups of 4 against 8, us: 32 experts, 2048 -> 512, 1920 slots (60 each) 937 /
+// 899, 128 experts (15 each) 924 / 985; 64 experts, 4096 -> 1024, 1920 slots (30
+// each) 2294 / 2412, 3840 (60 each) 4066 / 3793; 512 experts, 4096 -> 1024: 1920
+// slots 2480 / 2621, 3840: 4176 / 4212, 5000: 11513 / 10802 (an earlier build),
+// 7680: 7577 / 7304; 1024 experts, 2048 -> 512: 1920: 1011 / 1113, 7680: 2417 / 2424.
+int pf_iq2_cols(int n, int ne) { return n >= 1800 && (n >= 40 * ne || n >= 5000) ? 8 : 4; }
 // the most pieces of up to pf_iq2_cols slots of one expert that n slots make
-int pf_iq2_items(int n, int ne) { return n / pf_iq2_cols(n) + (ne < n ? ne : n); }
+int pf_iq2_items(int n, int ne) { return n / pf_iq2_cols(n, ne) + (ne < n ? ne : n); }
 
 bool pf_supported(const ornith_hip_model *m) {
     const ornith_hip_arch &a = m->a;
@@ -324,10 +341,11 @@ int pf_chunk(ornith_hip_session *s, int base, int T, bool chunked, hipStream_t s
                 // token t's j-th routed expert and reads token t's normalised
                 // row (and Q8_K planes) or its own silu(gate) * up
                 const Act ax = act_of(p.XQ, p.XN);
-                const bool gu = pf_iq2_slots(y.gate_exps, T * K) && pf_iq2_slots(y.up_exps, T * K) &&
+                const bool gu = pf_iq2_slots(y.gate_exps, T * K, a.ne) && pf_iq2_slots(y.up_exps, T * K, a.ne) &&
                                 y.up_exps->rows == y.gate_exps->rows && y.up_exps->in == y.gate_exps->in;
-                const bool dn = (gu || pairable(y.gate_exps, y.up_exps)) && pf_iq2_slots(y.down_exps, T * K);
-                const int cols = pf_iq2_cols(T * K), slot_items = pf_iq2_items(T * K, a.ne);
+                const bool dn = (gu || pairable(y.gate_exps, y.up_exps)) &&
+                                pf_iq2_slots(y.down_exps, T * K, a.ne);
+                const int cols = pf_iq2_cols(T * K, a.ne), slot_items = pf_iq2_items(T * K, a.ne);
                 if (gu || dn) HCHK(oh_launch_slot_lists(p.RIDX, T * K, a.ne, cols, p.CNT, p.LIST, p.ITEMS,
                                                             s->io + OH_IO_ERR, st));
                 Act ah;

@@ -6,6 +6,7 @@ its branches part and beside other types:
   with and without silu(gate) * up;
 * models whose gate and up projections are IQ2_XXS and whose down projections
   are not, and the reverse;
+* the sizes where the rule starts to group small experts that get few slots;
 * tokens that pick one expert twice (a router with NaN logits).
 
 Bar: the same bits as the oracle's rows, or as the token-by-token path."""
@@ -129,6 +130,24 @@ def test_mixed_expert_types_equal_token_path(hip_ctx, tmp_path, monkeypatch, iq2
     sp.free()
     st.free()
     m.free()
+
+
+@pytest.fixture(scope="module")
+def thin(hip_ctx):
+    m = hip_ctx.synth(**dict(IQ2X, n_layers=1, full_interval=2, ne=1024, top_k=8, moe_inter=256, shared_inter=256, seed=23))
+    yield m
+    m.free()
+
+
+@pytest.mark.parametrize("n", [59, 94, 95, 226])
+def test_small_thin_experts_equal_token_path(thin, monkeypatch, n):
+    """1024 experts of 768 -> 256, top 8: 472 and 752 slots keep the rows, 760
+    and 1808 (4 at a time: 1.8 slots an expert) are grouped."""
+    sp, st = both_paths(thin, np.random.default_rng(n).integers(0, thin.arch["vocab"], n).astype(np.int32), monkeypatch)
+    assert np.array_equal(u32(sp.logits()), u32(st.logits()))
+    same_state(thin, sp, st)
+    sp.free()
+    st.free()
 
 
 @pytest.mark.parametrize("ne", [8, 256])
