@@ -22,62 +22,15 @@ void seterr(const char *fmt, ...) {
 extern "C" const char *ornith_hip_last_error(void) { return g_err; }
 
 // ---- device memory ------------------------------------------------------------------
-// A session's buffers are parts of two or three blocks, and a closed session's
-// blocks serve the next session: a block of up to half again the size asked for
-// is taken. 4 GiB bounds what the pool holds (a 4096-token prompt's buffers of
-// the 35B shape take 1.5 GB); a model's end, a failed allocation and the
-// context's end give it back. Opening and closing a session allocated and freed
-// about 200 buffers before: a 4096-token request on 40 layers 131.5 -> 101.8 ms with
-// the pool, 1003 tokens on four layers 11.3 -> 4.1 ms.
-constexpr size_t kPoolBytes = (size_t)4 << 30, kPoolBlocks = 64;
+// (a failed allocation is returned, and not left for the next launch's check)
+static int hip_alloc(void **p, size_t n) {
+    const hipError_t e = hipMalloc(p, n);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return (int)e;
+}
+static void hip_release(void *p) { (void)hipFree(p); }
+DevMem hip_mem() { return {hip_alloc, hip_release}; }
 
-void dev_trim(ornith_hip_ctx *c) {
-    std::vector<DevBlock> old;
-    {
-        std::lock_guard<std::mutex> lk(c->pool_mu);
-        old.swap(c->pool);
-        c->pool_bytes = 0;
-    }
-    for (const DevBlock &b : old) (void)hipFree(b.p);
-}
-hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n) {
-    hipError_t e = hipMalloc(p, n);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();                  // the retry's status counts
-        dev_trim(c);
-        e = hipMalloc(p, n);
-    }
-    return e;
-}
-hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b) {
-    {
-        std::lock_guard<std::mutex> lk(c->pool_mu);
-        size_t best = c->pool.size();
-        for (size_t i = 0; i < c->pool.size(); i++) {
-            const size_t z = c->pool[i].n;
-            if (z >= n && z - n <= n / 2 + ((size_t)1 << 20) && (best == c->pool.size() || z < c->pool[best].n)) best = i;
-        }
-        if (best < c->pool.size()) {
-            *b = c->pool[best];
-            c->pool_bytes -= b->n;
-            c->pool.erase(c->pool.begin() + (ptrdiff_t)best);
-            return hipSuccess;
-        }
-    }
-    b->n = n;
-    return dev_malloc(c, &b->p, n);
-}
-void dev_put(ornith_hip_ctx *c, const DevBlock &b) {
-    {
-        std::lock_guard<std::mutex> lk(c->pool_mu);
-        if (c->pool_bytes + b.n <= kPoolBytes && c->pool.size() < kPoolBlocks) {
-            c->pool.push_back(b);
-            c->pool_bytes += b.n;
-            return;
-        }
-    }
-    (void)hipFree(b.p);
-}
 int sreserve(ornith_hip_session *s, size_t n) {
     ornith_hip_ctx *c = s->m->ctx;
     DevBlock b;
@@ -155,7 +108,6 @@ extern "C" void ornith_hip_free(ornith_hip_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->scratch) (void)hipFree(c->scratch);
-    dev_trim(c);
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
 }

@@ -27,6 +27,7 @@
 
 #include "../../include/ornith_hip.h"
 #include "oh_launch.h"
+#include "oh_pool.h"
 #include "oh_types.h"
 
 #define HCHK(call)                                                                    \
@@ -67,8 +68,7 @@ void seterr(const char *fmt, ...);
 
 
 // ---- context -----------------------------------------------------------------------
-// One device allocation of the context's pool (dev_get / dev_put).
-struct DevBlock { void *p = nullptr; size_t n = 0; };
+DevMem hip_mem();              // hipMalloc and hipFree
 
 struct ornith_hip_ctx {
     int device = 0;
@@ -77,17 +77,12 @@ struct ornith_hip_ctx {
     size_t scratch_bytes = 0;
     // allocations of closed sessions, kept for the next ones: work on them is
     // ordered by the context's one stream
-    std::mutex pool_mu;
-    std::vector<DevBlock> pool;
-    size_t pool_bytes = 0;
+    DevPool pool{hip_mem()};
 };
-// hipMalloc that gives the pool's blocks back and tries again when memory is short
-hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n);
-// a block of at least n bytes (contents undefined) from the pool or the device
-hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b);
-// the block back to the pool, or to the device beyond kPoolBytes
-void dev_put(ornith_hip_ctx *c, const DevBlock &b);
-void dev_trim(ornith_hip_ctx *c);
+inline hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n) { return (hipError_t)c->pool.alloc(p, n); }
+inline hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b) { return (hipError_t)c->pool.get(n, b); }
+inline void dev_put(ornith_hip_ctx *c, const DevBlock &b) { c->pool.put(b); }
+inline void dev_trim(ornith_hip_ctx *c) { c->pool.trim(); }
 
 // ---- tensors in the plane layout (oh_types.h) ---------------------------------------
 struct ornith_hip_tensor {

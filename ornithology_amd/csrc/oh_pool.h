@@ -1,0 +1,108 @@
+// oh_pool.h - device memory blocks kept between their users. The device's
+// memory calls are passed in, so this header holds no HIP.
+//
+// A session's buffers are parts of two or three blocks, and a closed session's
+// blocks serve the next session: a block of up to half again the size asked
+// for (and 1 MiB) is taken. Opening and closing a session allocated and freed
+// about 200 buffers before: a 4096-token request on 40 layers 131.5 -> 101.8 ms
+// with the pool, 1003 tokens on four layers 11.3 -> 4.1 ms.
+#pragma once
+#include <cstddef>
+#include <mutex>
+
+struct DevBlock { void *p = nullptr; size_t n = 0; };
+
+// The memory calls of a device.
+struct DevMem {
+    int (*alloc)(void **p, size_t n);     // 0, or the runtime's status
+    void (*release)(void *p);
+};
+
+class DevPool {
+public:
+    // What a pool holds at most (a 4096-token prompt's buffers of the 35B shape
+    // take 1.5 GB). Beyond it the blocks unused for longest are given back:
+    // sizes that no longer occur make room for those that do.
+    static constexpr size_t kBytes = (size_t)4 << 30;
+    static constexpr int kBlocks = 64;
+
+    explicit DevPool(const DevMem &mem) : mem_(mem) {}
+    ~DevPool() { trim(); }
+    DevPool(const DevPool &) = delete;
+    DevPool &operator=(const DevPool &) = delete;
+
+    // n bytes of device memory; when the device is out of it, once more after
+    // the pool's blocks are given back
+    int alloc(void **p, size_t n) {
+        int e = mem_.alloc(p, n);
+        if (e != 0) {
+            trim();
+            e = mem_.alloc(p, n);
+        }
+        return e;
+    }
+    // a block of at least n bytes (contents undefined) from the pool or the device
+    int get(size_t n, DevBlock *b) {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            int best = -1;
+            for (int i = 0; i < count_; i++) {
+                const size_t z = held_[i].n;
+                if (z >= n && z - n <= n / 2 + ((size_t)1 << 20) && (best < 0 || z < held_[best].n)) best = i;
+            }
+            if (best >= 0) {
+                *b = take(best);
+                return 0;
+            }
+        }
+        b->n = n;
+        return alloc(&b->p, n);
+    }
+    // the block back to the pool, or to the device when it is larger than the
+    // pool may be
+    void put(const DevBlock &b) {
+        if (b.n > kBytes) {
+            mem_.release(b.p);
+            return;
+        }
+        DevBlock old[kBlocks];
+        int n = 0;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            while (count_ == kBlocks || bytes_ + b.n > kBytes) old[n++] = take(0);
+            held_[count_++] = b;
+            bytes_ += b.n;
+        }
+        for (int i = 0; i < n; i++) mem_.release(old[i].p);
+    }
+    // all blocks back to the device; the bytes they held
+    size_t trim() {
+        DevBlock old[kBlocks];
+        int n = 0;
+        size_t bytes = 0;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            while (count_ > 0) old[n++] = take(count_ - 1);
+        }
+        for (int i = 0; i < n; i++) {
+            bytes += old[i].n;
+            mem_.release(old[i].p);
+        }
+        return bytes;
+    }
+
+private:
+    // held_[i] out of the pool (mu_ held)
+    DevBlock take(int i) {
+        const DevBlock b = held_[i];
+        bytes_ -= b.n;
+        for (count_--; i < count_; i++) held_[i] = held_[i + 1];
+        return b;
+    }
+
+    DevMem mem_;
+    std::mutex mu_;
+    DevBlock held_[kBlocks];              // unused for longest first
+    int count_ = 0;
+    size_t bytes_ = 0;
+};

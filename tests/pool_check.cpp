@@ -1,0 +1,138 @@
+// Checks of ornithology_amd/csrc/oh_pool.h over a made-up device: one check per
+// run, named by the first argument (tests/test_pool.py builds and runs them).
+#include "oh_pool.h"
+
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+
+namespace {
+
+constexpr size_t MiB = (size_t)1 << 20, GiB = (size_t)1 << 30;
+size_t capacity = 288 * GiB, used = 0;
+uintptr_t next_addr = 0x1000;
+std::map<void *, size_t> live;
+int allocs = 0;
+
+int dev_alloc(void **p, size_t n) {
+    if (used + n > capacity) return 2;
+    *p = (void *)next_addr;
+    next_addr += n + 256;
+    live[*p] = n;
+    used += n;
+    allocs++;
+    return 0;
+}
+void dev_release(void *p) {
+    auto it = live.find(p);
+    if (it == live.end()) {
+        printf("a block that is not live was released\n");
+        exit(1);
+    }
+    used -= it->second;
+    live.erase(it);
+}
+const DevMem kMem = {dev_alloc, dev_release};
+
+#define CHECK(x)                                                     \
+    do {                                                             \
+        if (!(x)) {                                                  \
+            printf("%s:%d: %s\n", __FILE__, __LINE__, #x);           \
+            return 1;                                                \
+        }                                                            \
+    } while (0)
+
+DevBlock get(DevPool &p, size_t n) {
+    DevBlock b;
+    if (p.get(n, &b) != 0) {
+        printf("no block of %zu bytes\n", n);
+        exit(1);
+    }
+    return b;
+}
+
+// a block serves sizes down to two thirds of it (and 1 MiB), the smallest such one
+int fit() {
+    DevPool p(kMem);
+    const DevBlock a = get(p, 300 * MiB), b = get(p, 290 * MiB);
+    p.put(a);
+    p.put(b);
+    CHECK(get(p, 301 * MiB).p != a.p);
+    const DevBlock c = get(p, 250 * MiB);
+    CHECK(c.p == b.p && c.n == b.n);
+    CHECK(get(p, 150 * MiB).p != a.p);
+    CHECK(get(p, 200 * MiB).p == a.p);
+    return 0;
+}
+
+// sizes that no longer occur do not keep those that do out of the pool
+int unusable_bytes() {
+    DevPool p(kMem);
+    DevBlock b[4];
+    for (int i = 0; i < 4; i++) b[i] = get(p, (size_t)(10 + i) * GiB / 13);
+    for (const DevBlock &x : b) p.put(x);
+    const DevBlock s = get(p, 2 * GiB);
+    p.put(s);
+    CHECK(get(p, 2 * GiB).p == s.p);
+    CHECK(used <= 6 * GiB);
+    return 0;
+}
+int unusable_blocks() {
+    DevPool p(kMem);
+    DevBlock b[3 * DevPool::kBlocks];
+    for (int i = 0; i < 3 * DevPool::kBlocks; i++) b[i] = get(p, 4096 + 256 * i);
+    for (const DevBlock &x : b) p.put(x);
+    CHECK((int)live.size() == DevPool::kBlocks);
+    const DevBlock s = get(p, 64 * MiB);
+    p.put(s);
+    CHECK((int)live.size() == DevPool::kBlocks);
+    CHECK(get(p, 64 * MiB).p == s.p);
+    return 0;
+}
+
+// the pool never holds more than its bounds, and gives the oldest back first
+int bounds() {
+    DevPool p(kMem);
+    DevBlock b[8];
+    for (int i = 0; i < 8; i++) b[i] = get(p, GiB);
+    for (const DevBlock &x : b) {
+        p.put(x);
+        CHECK(live.count(x.p) == 1);
+    }
+    CHECK(used == DevPool::kBytes);
+    for (int i = 0; i < 8; i++) CHECK(live.count(b[i].p) == (i >= 4 ? 1u : 0u));
+    const DevBlock big = get(p, DevPool::kBytes + 1);
+    p.put(big);
+    CHECK(live.count(big.p) == 0 && used == DevPool::kBytes);
+    CHECK(p.trim() == DevPool::kBytes && used == 0 && p.trim() == 0);
+    return 0;
+}
+
+// an allocation that fails is tried again without the pool's blocks
+int retry() {
+    DevPool p(kMem);
+    capacity = 8 * GiB;
+    const DevBlock a = get(p, 3 * GiB);
+    p.put(a);
+    CHECK(used == 3 * GiB);
+    void *q = nullptr;
+    CHECK(p.alloc(&q, 6 * GiB) == 0 && used == 6 * GiB && live.count(a.p) == 0);
+    CHECK(p.alloc(&q, 3 * GiB) == 2 && used == 6 * GiB);
+    return 0;
+}
+
+const struct { const char *name; int (*run)(); } kChecks[] = {
+    {"fit", fit}, {"unusable_bytes", unusable_bytes}, {"unusable_blocks", unusable_blocks},
+    {"bounds", bounds}, {"retry", retry},
+};
+
+} // namespace
+
+int main(int argc, char **argv) {
+    for (const auto &c : kChecks)
+        if (argc > 1 && strcmp(argv[1], c.name) == 0) return c.run();
+    printf("no such check\n");
+    return 2;
+}
