@@ -75,6 +75,8 @@ typedef struct {
 const char *ornith_hip_last_error(void);            /* ornith_last_error, src/ornith_util.c:25-30 */
 
 int  ornith_hip_init(int device, ornith_hip_ctx **out);
+/* Models and sessions may be freed before or after their context, and sessions
+ * after their model; the context's stream and memory go with the last of them. */
 void ornith_hip_free(ornith_hip_ctx *ctx);
 int  ornith_hip_sync(ornith_hip_ctx *ctx);            /* wait for all work on the device */
 

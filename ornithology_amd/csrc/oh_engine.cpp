@@ -105,7 +105,10 @@ extern "C" int ornith_hip_sync(ornith_hip_ctx *c) {
 }
 
 extern "C" void ornith_hip_free(ornith_hip_ctx *c) {
-    if (!c) return;
+    if (c) ctx_drop(c);
+}
+void ctx_drop(ornith_hip_ctx *c) {
+    if (--c->refs > 0) return;
     (void)hipSetDevice(c->device);
     if (c->scratch) (void)hipFree(c->scratch);
     if (c->st) (void)hipStreamDestroy(c->st);

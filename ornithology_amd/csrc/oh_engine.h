@@ -78,6 +78,18 @@ struct ornith_hip_ctx {
     // allocations of closed sessions, kept for the next ones: work on them is
     // ordered by the context's one stream
     DevPool pool{hip_mem()};
+    // the caller's handle, and the models and sessions, whose end uses the
+    // stream and the pool: the last of them ends the context
+    std::atomic<int> refs{1};
+};
+void ctx_drop(ornith_hip_ctx *c);
+struct CtxRef {
+    ornith_hip_ctx *c = nullptr;
+    CtxRef() = default;
+    CtxRef(const CtxRef &) = delete;
+    CtxRef &operator=(const CtxRef &) = delete;
+    void hold(ornith_hip_ctx *ctx) { c = ctx; c->refs++; }
+    ~CtxRef() { if (c) ctx_drop(c); }
 };
 inline hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n) { return (hipError_t)c->pool.alloc(p, n); }
 inline hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b) { return (hipError_t)c->pool.get(n, b); }
@@ -140,6 +152,7 @@ struct OhLayer {
 
 struct ornith_hip_model {
     ornith_hip_ctx *ctx = nullptr;
+    CtxRef ref;
     ornith_hip_arch a;
     std::vector<ornith_hip_tensor *> ts;
     std::unordered_map<std::string, ornith_hip_tensor *> by;
@@ -177,6 +190,7 @@ struct LayerState {
 
 struct ornith_hip_session {
     ornith_hip_model *m = nullptr;
+    CtxRef ref;                   // (the model may be freed before the session)
     uint64_t sid = 0;             // unique per session of the process
     int cap = 0, pos = 0, kvcap = 0;
     bool have_logits = false;

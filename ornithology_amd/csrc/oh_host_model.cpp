@@ -271,6 +271,7 @@ extern "C" int ornith_hip_model_load(ornith_hip_ctx *ctx, const char *path, orni
     if (ie != g.kv.end() && ie->second.len >= 4) memcpy(&md.eos, ie->second.val, 4);
     auto *m = new ornith_hip_model();
     m->ctx = ctx;
+    m->ref.hold(ctx);
     for (auto &t : g.ts) {
         ornith_hip_tensor *dt;
         int st = ornith_hip_upload(ctx, t.name.c_str(), t.type, t.data, t.nbytes, t.nd, t.dims, &dt);

@@ -63,12 +63,13 @@ void prog_mv(Prog &P, MvBuild &b) {
 
 extern "C" void ornith_hip_session_free(ornith_hip_session *s) {
     if (!s) return;
-    (void)hipSetDevice(s->m->ctx->device);
+    ornith_hip_ctx *c = s->ref.c;
+    (void)hipSetDevice(c->device);
     if (s->gbody) (void)hipGraphExecDestroy(s->gbody);
     if (s->gbody_x) (void)hipGraphExecDestroy(s->gbody_x);
     if (s->ghead) (void)hipGraphExecDestroy(s->ghead);
     if (s->bw.graph) (void)hipGraphExecDestroy(s->bw.graph);
-    for (const DevBlock &b : s->blocks) dev_put(s->m->ctx, b);
+    for (const DevBlock &b : s->blocks) dev_put(c, b);
     delete s;
 }
 int q8alloc(ornith_hip_session *s, Q8Buf &q, size_t n) {
@@ -145,6 +146,7 @@ extern "C" int ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_s
     static std::atomic<uint64_t> next_sid{1};
     s->sid = next_sid++;
     s->m = m;
+    s->ref.hold(m->ctx);
     s->cap = cap;
     s->kvcap = (cap + 15) / 16 * 16;   // KV storage stride (V is tiled by 16 positions)
     const int H = a.hidden, qd = a.nk * a.dk, vd = a.nv * a.dv, cc = 2 * qd + vd;
