@@ -80,8 +80,7 @@ extern "C" int ornith_hip_init(int device, ornith_hip_ctx **out) {
         return ORNITH_HIP_ERR_NOTFOUND;
     }
     HCHK(hipSetDevice(device));
-    auto *c = new ornith_hip_ctx();
-    c->device = device;
+    auto *c = new ornith_hip_ctx(device);
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
     if (e != hipSuccess) {
         delete c;

@@ -71,13 +71,14 @@ void seterr(const char *fmt, ...);
 DevMem hip_mem();              // hipMalloc and hipFree
 
 struct ornith_hip_ctx {
-    int device = 0;
+    explicit ornith_hip_ctx(int device) : device(device), pool(hip_mem(), device) {}
+    const int device;
     hipStream_t st = nullptr;
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
     // allocations of closed sessions, kept for the next ones: work on them is
     // ordered by the context's one stream
-    DevPool pool{hip_mem()};
+    DevPool pool;
     // the caller's handle, and the models and sessions, whose end uses the
     // stream and the pool: the last of them ends the context
     std::atomic<int> refs{1};

@@ -26,17 +26,33 @@ public:
     static constexpr size_t kBytes = (size_t)4 << 30;
     static constexpr int kBlocks = 64;
 
-    explicit DevPool(const DevMem &mem) : mem_(mem) {}
-    ~DevPool() { trim(); }
+    DevPool(const DevMem &mem, int device) : mem_(mem), device_(device) {
+        std::lock_guard<std::mutex> lk(all_mu());
+        next_ = all();
+        all() = this;
+    }
+    ~DevPool() {
+        {
+            std::lock_guard<std::mutex> lk(all_mu());
+            DevPool **p = &all();
+            while (*p != this) p = &(*p)->next_;
+            *p = next_;
+        }
+        trim();
+    }
     DevPool(const DevPool &) = delete;
     DevPool &operator=(const DevPool &) = delete;
 
     // n bytes of device memory; when the device is out of it, once more after
-    // the pool's blocks are given back
+    // the blocks of all of the device's pools are given back
     int alloc(void **p, size_t n) {
         int e = mem_.alloc(p, n);
         if (e != 0) {
-            trim();
+            {
+                std::lock_guard<std::mutex> lk(all_mu());
+                for (DevPool *q = all(); q; q = q->next_)
+                    if (q->device_ == device_) q->trim();
+            }
             e = mem_.alloc(p, n);
         }
         return e;
@@ -92,6 +108,10 @@ public:
     }
 
 private:
+    // the process's pools
+    static DevPool *&all() { static DevPool *head = nullptr; return head; }
+    static std::mutex &all_mu() { static std::mutex m; return m; }
+
     // held_[i] out of the pool (mu_ held)
     DevBlock take(int i) {
         const DevBlock b = held_[i];
@@ -101,6 +121,8 @@ private:
     }
 
     DevMem mem_;
+    int device_;
+    DevPool *next_ = nullptr;
     std::mutex mu_;
     DevBlock held_[kBlocks];              // unused for longest first
     int count_ = 0;

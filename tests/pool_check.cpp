@@ -55,7 +55,7 @@ DevBlock get(DevPool &p, size_t n) {
 
 // a block serves sizes down to two thirds of it (and 1 MiB), the smallest such one
 int fit() {
-    DevPool p(kMem);
+    DevPool p(kMem, 0);
     const DevBlock a = get(p, 300 * MiB), b = get(p, 290 * MiB);
     p.put(a);
     p.put(b);
@@ -69,7 +69,7 @@ int fit() {
 
 // sizes that no longer occur do not keep those that do out of the pool
 int unusable_bytes() {
-    DevPool p(kMem);
+    DevPool p(kMem, 0);
     DevBlock b[4];
     for (int i = 0; i < 4; i++) b[i] = get(p, (size_t)(10 + i) * GiB / 13);
     for (const DevBlock &x : b) p.put(x);
@@ -80,7 +80,7 @@ int unusable_bytes() {
     return 0;
 }
 int unusable_blocks() {
-    DevPool p(kMem);
+    DevPool p(kMem, 0);
     DevBlock b[3 * DevPool::kBlocks];
     for (int i = 0; i < 3 * DevPool::kBlocks; i++) b[i] = get(p, 4096 + 256 * i);
     for (const DevBlock &x : b) p.put(x);
@@ -94,7 +94,7 @@ int unusable_blocks() {
 
 // the pool never holds more than its bounds, and gives the oldest back first
 int bounds() {
-    DevPool p(kMem);
+    DevPool p(kMem, 0);
     DevBlock b[8];
     for (int i = 0; i < 8; i++) b[i] = get(p, GiB);
     for (const DevBlock &x : b) {
@@ -112,7 +112,7 @@ int bounds() {
 
 // an allocation that fails is tried again without the pool's blocks
 int retry() {
-    DevPool p(kMem);
+    DevPool p(kMem, 0);
     capacity = 8 * GiB;
     const DevBlock a = get(p, 3 * GiB);
     p.put(a);
@@ -123,9 +123,26 @@ int retry() {
     return 0;
 }
 
+// ... and without those of the device's other pools; another device's stay
+int other_pools() {
+    DevPool p(kMem, 0), other(kMem, 1);
+    auto *q = new DevPool(kMem, 0);
+    capacity = 8 * GiB;
+    const DevBlock a = get(p, GiB), b = get(*q, 2 * GiB), c = get(other, GiB);
+    p.put(a);
+    q->put(b);
+    other.put(c);
+    void *x = nullptr;
+    CHECK(p.alloc(&x, 6 * GiB) == 0);
+    CHECK(live.count(a.p) == 0 && live.count(b.p) == 0 && live.count(c.p) == 1);
+    delete q;
+    CHECK(p.alloc(&x, 2 * GiB) == 2 && live.count(c.p) == 1);
+    return 0;
+}
+
 const struct { const char *name; int (*run)(); } kChecks[] = {
     {"fit", fit}, {"unusable_bytes", unusable_bytes}, {"unusable_blocks", unusable_blocks},
-    {"bounds", bounds}, {"retry", retry},
+    {"bounds", bounds}, {"retry", retry}, {"other_pools", other_pools},
 };
 
 } // namespace
