@@ -158,7 +158,12 @@ const ornith_hip_tensor *ornith_hip_model_tensor(const ornith_hip_model *m, cons
  * Q6_K tensors the prompt runs on the matrix cores, about their GGUF size;
  * none with ORNITH_HIP_MMQ=0); they are freed with the model. */
 int  ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_session **out);
-void ornith_hip_session_free(ornith_hip_session *s);                             /* rmodel_session_free */
+/* rmodel_session_free. The context keeps the device memory of closed sessions
+ * (and of ornith_hip_quantize) for the next ones: up to 4 GiB, and up to a
+ * sixteenth of what the device has unused otherwise; the part unused for
+ * longest is given back first. A call of this library that finds no memory
+ * takes it back, from every context on the device. */
+void ornith_hip_session_free(ornith_hip_session *s);
 /* rmodel_session_eval (src/ornith_rforward.c:838-849,933-944): the prompt runs
  * layer by layer over engine chunks of up to 4096 tokens (ORNITH_HIP_PREFILL_CHUNK,
  * a multiple of 32; the chunk length changes no result bit) with batched

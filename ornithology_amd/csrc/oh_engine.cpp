@@ -29,7 +29,12 @@ static int hip_alloc(void **p, size_t n) {
     return (int)e;
 }
 static void hip_release(void *p) { (void)hipFree(p); }
-DevMem hip_mem() { return {hip_alloc, hip_release}; }
+static size_t hip_unused(int device) {
+    size_t unused = 0, total = 0;
+    if (hipSetDevice(device) != hipSuccess || hipMemGetInfo(&unused, &total) != hipSuccess) return 0;
+    return unused;
+}
+DevMem hip_mem() { return {hip_alloc, hip_release, hip_unused}; }
 
 int sreserve(ornith_hip_session *s, size_t n) {
     ornith_hip_ctx *c = s->m->ctx;

@@ -68,7 +68,7 @@ void seterr(const char *fmt, ...);
 
 
 // ---- context -----------------------------------------------------------------------
-DevMem hip_mem();              // hipMalloc and hipFree
+DevMem hip_mem();              // hipMalloc, hipFree, hipMemGetInfo
 
 struct ornith_hip_ctx {
     explicit ornith_hip_ctx(int device) : device(device), pool(hip_mem(), device) {}

@@ -16,14 +16,17 @@ struct DevBlock { void *p = nullptr; size_t n = 0; };
 struct DevMem {
     int (*alloc)(void **p, size_t n);     // 0, or the runtime's status
     void (*release)(void *p);
+    size_t (*unused)(int device);         // bytes of the device that nobody holds
 };
 
 class DevPool {
 public:
     // What a pool holds at most (a 4096-token prompt's buffers of the 35B shape
-    // take 1.5 GB). Beyond it the blocks unused for longest are given back:
-    // sizes that no longer occur make room for those that do.
-    static constexpr size_t kBytes = (size_t)4 << 30;
+    // take 1.5 GB), and at most this share of the memory that is not in use
+    // otherwise: other users of the device see what is held as taken. Beyond it
+    // the blocks unused for longest are given back: sizes that no longer occur
+    // make room for those that do. (Asking the device takes 5 us a block.)
+    static constexpr size_t kBytes = (size_t)4 << 30, kShare = 16;
     static constexpr int kBlocks = 64;
 
     DevPool(const DevMem &mem, int device) : mem_(mem), device_(device) {
@@ -74,20 +77,23 @@ public:
         b->n = n;
         return alloc(&b->p, n);
     }
-    // the block back to the pool, or to the device when it is larger than the
-    // pool may be
+    // the block back to the pool, or to the device when the pool may not be
+    // that large
     void put(const DevBlock &b) {
-        if (b.n > kBytes) {
-            mem_.release(b.p);
-            return;
-        }
-        DevBlock old[kBlocks];
+        const size_t unused = mem_.unused(device_);
+        DevBlock old[kBlocks + 1];
         int n = 0;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            while (count_ == kBlocks || bytes_ + b.n > kBytes) old[n++] = take(0);
-            held_[count_++] = b;
-            bytes_ += b.n;
+            const size_t share = (unused + bytes_ + b.n) / kShare, most = share < kBytes ? share : kBytes;
+            const bool keep = b.n <= most;
+            while ((keep && count_ == kBlocks) || (count_ > 0 && bytes_ + (keep ? b.n : 0) > most)) old[n++] = take(0);
+            if (keep) {
+                held_[count_++] = b;
+                bytes_ += b.n;
+            } else {
+                old[n++] = b;
+            }
         }
         for (int i = 0; i < n; i++) mem_.release(old[i].p);
     }

@@ -34,7 +34,8 @@ void dev_release(void *p) {
     used -= it->second;
     live.erase(it);
 }
-const DevMem kMem = {dev_alloc, dev_release};
+size_t dev_unused(int) { return capacity - used; }
+const DevMem kMem = {dev_alloc, dev_release, dev_unused};
 
 #define CHECK(x)                                                     \
     do {                                                             \
@@ -110,13 +111,31 @@ int bounds() {
     return 0;
 }
 
+// on a device that is nearly full the pool keeps a sixteenth of the rest
+int share() {
+    DevPool p(kMem, 0);
+    capacity = 100 * GiB;
+    const DevBlock a = get(p, 2 * GiB), s = get(p, 100 * MiB);
+    p.put(a);
+    const DevBlock rest = get(p, 93 * GiB);
+    CHECK(live.count(a.p) == 1);
+    p.put(s);                              // 7 GiB without it and a: room for 448 MiB
+    CHECK(live.count(a.p) == 0 && live.count(s.p) == 1);
+    const DevBlock c = get(p, GiB);
+    p.put(c);
+    CHECK(live.count(c.p) == 0 && live.count(s.p) == 1);
+    p.put(get(p, 300 * MiB));
+    CHECK(live.count(s.p) == 1 && used == rest.n + 400 * MiB);
+    return 0;
+}
+
 // an allocation that fails is tried again without the pool's blocks
 int retry() {
     DevPool p(kMem, 0);
-    capacity = 8 * GiB;
     const DevBlock a = get(p, 3 * GiB);
     p.put(a);
     CHECK(used == 3 * GiB);
+    capacity = 8 * GiB;
     void *q = nullptr;
     CHECK(p.alloc(&q, 6 * GiB) == 0 && used == 6 * GiB && live.count(a.p) == 0);
     CHECK(p.alloc(&q, 3 * GiB) == 2 && used == 6 * GiB);
@@ -127,11 +146,11 @@ int retry() {
 int other_pools() {
     DevPool p(kMem, 0), other(kMem, 1);
     auto *q = new DevPool(kMem, 0);
-    capacity = 8 * GiB;
     const DevBlock a = get(p, GiB), b = get(*q, 2 * GiB), c = get(other, GiB);
     p.put(a);
     q->put(b);
     other.put(c);
+    capacity = 8 * GiB;
     void *x = nullptr;
     CHECK(p.alloc(&x, 6 * GiB) == 0);
     CHECK(live.count(a.p) == 0 && live.count(b.p) == 0 && live.count(c.p) == 1);
@@ -142,7 +161,7 @@ int other_pools() {
 
 const struct { const char *name; int (*run)(); } kChecks[] = {
     {"fit", fit}, {"unusable_bytes", unusable_bytes}, {"unusable_blocks", unusable_blocks},
-    {"bounds", bounds}, {"retry", retry}, {"other_pools", other_pools},
+    {"bounds", bounds}, {"share", share}, {"retry", retry}, {"other_pools", other_pools},
 };
 
 } // namespace
