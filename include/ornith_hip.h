@@ -161,7 +161,8 @@ int  ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_session **o
 /* rmodel_session_free. The context keeps the device memory of closed sessions
  * (and of ornith_hip_quantize) for the next ones: up to 4 GiB, and up to a
  * sixteenth of what the device has unused otherwise; the part unused for
- * longest is given back first. A call of this library that finds no memory
+ * longest is given back first, and a model's end gives back what its sessions
+ * held. A call of this library that finds no memory
  * takes it back, from every context on the device. */
 void ornith_hip_session_free(ornith_hip_session *s);
 /* rmodel_session_eval (src/ornith_rforward.c:838-849,933-944): the prompt runs

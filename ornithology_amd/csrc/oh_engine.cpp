@@ -40,6 +40,7 @@ int sreserve(ornith_hip_session *s, size_t n) {
     ornith_hip_ctx *c = s->m->ctx;
     DevBlock b;
     HCHK(dev_get(c, n, &b));
+    b.owner = s->m;
     s->blocks.push_back(b);
     HCHK(hipMemsetAsync(b.p, 0, n, c->st));
     HCHK(hipStreamSynchronize(c->st));            // copies that are not on the stream may follow

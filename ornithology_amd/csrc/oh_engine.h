@@ -95,7 +95,6 @@ struct CtxRef {
 inline hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n) { return (hipError_t)c->pool.alloc(p, n); }
 inline hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b) { return (hipError_t)c->pool.get(n, b); }
 inline void dev_put(ornith_hip_ctx *c, const DevBlock &b) { c->pool.put(b); }
-inline void dev_trim(ornith_hip_ctx *c) { c->pool.trim(); }
 
 // ---- tensors in the plane layout (oh_types.h) ---------------------------------------
 struct ornith_hip_tensor {

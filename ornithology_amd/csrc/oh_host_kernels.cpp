@@ -195,6 +195,7 @@ extern "C" int ornith_hip_quantize(ornith_hip_ctx *ctx, uint32_t type, const flo
     DevBlock blk;
     hipError_t e = dev_get(ctx, up256(pa) + up256(pb) + up256(pc) + n * 4, &blk);
     if (e != hipSuccess) { seterr("quantize: %s", hipGetErrorString(e)); return ORNITH_HIP_ERR_OOM; }
+    blk.owner = nullptr;
     uint8_t *A = (uint8_t *)blk.p, *B = A + up256(pa), *C = B + up256(pb);
     float *dx = (float *)(C + up256(pc));
     e = hipMemcpyAsync(dx, x, n * 4, hipMemcpyHostToDevice, ctx->st);

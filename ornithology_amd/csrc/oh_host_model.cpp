@@ -115,7 +115,7 @@ extern "C" void ornith_hip_model_free(ornith_hip_model *m) {
     if (!m) return;
     for (auto *t : m->ts) ornith_hip_tensor_free(t);
     for (float2 *r : m->rope_all) (void)hipFree(r);
-    dev_trim(m->ctx);                             // closed sessions' memory goes with the model
+    m->ctx->pool.trim(m);                         // its closed sessions' memory goes with the model
     delete m;
 }
 

@@ -10,7 +10,11 @@
 #include <cstddef>
 #include <mutex>
 
-struct DevBlock { void *p = nullptr; size_t n = 0; };
+struct DevBlock {
+    void *p = nullptr;
+    size_t n = 0;
+    const void *owner = nullptr;          // whom it served last (a model; null: none in particular)
+};
 
 // The memory calls of a device.
 struct DevMem {
@@ -97,14 +101,16 @@ public:
         }
         for (int i = 0; i < n; i++) mem_.release(old[i].p);
     }
-    // all blocks back to the device; the bytes they held
-    size_t trim() {
+    // all blocks back to the device, or those that served owner last; the bytes
+    // they held
+    size_t trim(const void *owner = nullptr) {
         DevBlock old[kBlocks];
         int n = 0;
         size_t bytes = 0;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            while (count_ > 0) old[n++] = take(count_ - 1);
+            for (int i = count_ - 1; i >= 0; i--)
+                if (!owner || held_[i].owner == owner) old[n++] = take(i);
         }
         for (int i = 0; i < n; i++) {
             bytes += old[i].n;

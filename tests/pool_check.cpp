@@ -129,6 +129,24 @@ int share() {
     return 0;
 }
 
+// the end of one user leaves the blocks that served others
+int owners() {
+    DevPool p(kMem, 0);
+    int one, two;
+    DevBlock a = get(p, 10 * MiB), b = get(p, 20 * MiB), c = get(p, 40 * MiB), d = get(p, 80 * MiB);
+    a.owner = c.owner = &one;
+    b.owner = &two;
+    for (const DevBlock &x : {a, b, c, d}) p.put(x);
+    CHECK(p.trim(&one) == 50 * MiB);
+    CHECK(live.count(a.p) == 0 && live.count(c.p) == 0 && live.count(b.p) == 1 && live.count(d.p) == 1);
+    DevBlock e = get(p, 20 * MiB);
+    CHECK(e.p == b.p);
+    e.owner = &one;                       // now it serves the other one
+    p.put(e);
+    CHECK(p.trim(&two) == 0 && p.trim(&one) == 20 * MiB && p.trim() == 80 * MiB);
+    return 0;
+}
+
 // an allocation that fails is tried again without the pool's blocks
 int retry() {
     DevPool p(kMem, 0);
@@ -161,7 +179,7 @@ int other_pools() {
 
 const struct { const char *name; int (*run)(); } kChecks[] = {
     {"fit", fit}, {"unusable_bytes", unusable_bytes}, {"unusable_blocks", unusable_blocks},
-    {"bounds", bounds}, {"share", share}, {"retry", retry}, {"other_pools", other_pools},
+    {"bounds", bounds}, {"share", share}, {"owners", owners}, {"retry", retry}, {"other_pools", other_pools},
 };
 
 } // namespace
