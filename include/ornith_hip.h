@@ -79,6 +79,10 @@ int  ornith_hip_init(int device, ornith_hip_ctx **out);
  * after their model; the context's stream and memory go with the last of them. */
 void ornith_hip_free(ornith_hip_ctx *ctx);
 int  ornith_hip_sync(ornith_hip_ctx *ctx);            /* wait for all work on the device */
+/* Give the device memory that the context keeps between calls (see
+ * ornith_hip_session_free) back to the device; *bytes (may be NULL): how much
+ * it was. No reference twin. */
+int  ornith_hip_trim(ornith_hip_ctx *ctx, uint64_t *bytes);
 
 /* ---- ornith_qdot / codecs (kernel-level boundary) --------------------------- */
 
@@ -163,7 +167,8 @@ int  ornith_hip_session_new(ornith_hip_model *m, int cap, ornith_hip_session **o
  * sixteenth of what the device has unused otherwise; the part unused for
  * longest is given back first, and a model's end gives back what its sessions
  * held. A call of this library that finds no memory
- * takes it back, from every context on the device. */
+ * takes it back, from every context on the device; before other libraries
+ * need it, ornith_hip_trim does. */
 void ornith_hip_session_free(ornith_hip_session *s);
 /* rmodel_session_eval (src/ornith_rforward.c:838-849,933-944): the prompt runs
  * layer by layer over engine chunks of up to 4096 tokens (ORNITH_HIP_PREFILL_CHUNK,

@@ -63,6 +63,7 @@ _SIGS = {
     "ornith_hip_init": (C.c_int, [C.c_int, C.POINTER(_vp)]),
     "ornith_hip_free": (None, [_vp]),
     "ornith_hip_sync": (C.c_int, [_vp]),
+    "ornith_hip_trim": (C.c_int, [_vp, C.POINTER(C.c_uint64)]),
     "ornith_hip_upload": (C.c_int, [_vp, C.c_char_p, C.c_uint32, _vp, C.c_uint64, C.c_uint32,
                                     C.POINTER(C.c_uint64), C.POINTER(_vp)]),
     "ornith_hip_tensor_free": (None, [_vp]),
@@ -151,6 +152,12 @@ class Context:
 
     def sync(self) -> None:
         _check(lib().ornith_hip_sync(self.h), "ornith_hip_sync")
+
+    def trim(self) -> int:
+        """Give back the device memory kept from closed sessions; the bytes."""
+        n = C.c_uint64(0)
+        _check(lib().ornith_hip_trim(self.h, C.byref(n)), "ornith_hip_trim")
+        return n.value
 
     def close(self):
         if self.h:

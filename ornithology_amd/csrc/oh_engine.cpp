@@ -109,6 +109,13 @@ extern "C" int ornith_hip_sync(ornith_hip_ctx *c) {
     return ORNITH_HIP_OK;
 }
 
+extern "C" int ornith_hip_trim(ornith_hip_ctx *c, uint64_t *bytes) {
+    HCHK(hipSetDevice(c->device));
+    const size_t n = c->pool.trim();
+    if (bytes) *bytes = n;
+    return ORNITH_HIP_OK;
+}
+
 extern "C" void ornith_hip_free(ornith_hip_ctx *c) {
     if (c) ctx_drop(c);
 }

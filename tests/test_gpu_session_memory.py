@@ -1,7 +1,9 @@
 """GPU: sessions opened on a closed session's memory (the context keeps it for
 the next one). A session that takes over the blocks of a larger, a smaller or an
 equal one, with other sessions open beside it, gives the bits that a session on
-fresh memory gives: prompt logits, greedy tokens and state."""
+fresh memory gives: prompt logits, greedy tokens and state. What the context
+keeps is one session's memory however many were opened in turn, and
+Context.trim gives it back."""
 import numpy as np
 import pytest
 
@@ -44,4 +46,46 @@ def test_sessions_on_reused_memory(monkeypatch):
             held = s                      # one session stays open beside the next
     held.free()
     m.free()
+    ctx.close()
+
+
+def test_closed_sessions_memory_serves_the_next():
+    ctx = oa.Context(0)
+    m = ctx.synth(**clibs.C1)
+    p = np.random.default_rng(6).integers(0, clibs.C1["vocab"], 500).astype(np.int32)
+
+    def kept(caps, n=500):
+        for cap in caps:
+            s = m.session(cap)
+            s.eval(p[:n])
+            s.free()
+        return ctx.trim()
+
+    kept([4000])
+    one = kept([4000])
+    assert one > 4000 * 2 * (64 + 4)          # the KV codes and scales of one KV head at least
+    assert ctx.trim() == 0
+    assert kept([4000] * 6) == one            # each took the one before it's
+    assert kept([4000, 3500, 3900, 4000]) == one
+    assert kept([4000, 64000]) > one          # too small for the next: both are kept
+    a, b = m.session(4000), m.session(4000)   # open together: no memory in common
+    a.eval(p)
+    b.eval(p)
+    a.free()
+    b.free()
+    assert kept([4000]) == 2 * one
+    x = clibs.gauss(8, "kept", 256 * 4096)
+    ctx.quantize(clibs.Q4_K, x)
+    enc = ctx.trim()
+    assert enc >= x.nbytes
+    for _ in range(3):
+        ctx.quantize(clibs.Q4_K, x)
+    assert ctx.trim() == enc
+    kept([4000])
+    m.free()                                  # gives back what its sessions held
+    assert ctx.trim() == 0
+    m = ctx.synth(**clibs.C1)
+    m.session(4000).free()
+    m.free()
+    assert ctx.trim() == 0
     ctx.close()
