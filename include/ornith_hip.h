@@ -80,8 +80,9 @@ int  ornith_hip_init(int device, ornith_hip_ctx **out);
 void ornith_hip_free(ornith_hip_ctx *ctx);
 int  ornith_hip_sync(ornith_hip_ctx *ctx);            /* wait for all work on the device */
 /* Give the device memory that the context keeps between calls (see
- * ornith_hip_session_free) back to the device; *bytes (may be NULL): how much
- * it was. No reference twin. */
+ * ornith_hip_session_free; also each model's RoPE table for its longest session
+ * so far, while no session reads it) back to the device; *bytes (may be NULL):
+ * how much it was. No reference twin. */
 int  ornith_hip_trim(ornith_hip_ctx *ctx, uint64_t *bytes);
 
 /* ---- ornith_qdot / codecs (kernel-level boundary) --------------------------- */

@@ -111,7 +111,7 @@ extern "C" int ornith_hip_sync(ornith_hip_ctx *c) {
 
 extern "C" int ornith_hip_trim(ornith_hip_ctx *c, uint64_t *bytes) {
     HCHK(hipSetDevice(c->device));
-    const size_t n = c->pool.trim();
+    const size_t n = c->pool.trim() + trim_tables(c);
     if (bytes) *bytes = n;
     return ORNITH_HIP_OK;
 }

@@ -8,12 +8,14 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <algorithm>
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <cstring>
 #include <string>
@@ -79,6 +81,8 @@ struct ornith_hip_ctx {
     // allocations of closed sessions, kept for the next ones: work on them is
     // ordered by the context's one stream
     DevPool pool;
+    std::mutex models_mu;
+    std::vector<ornith_hip_model *> models;
     // the caller's handle, and the models and sessions, whose end uses the
     // stream and the pool: the last of them ends the context
     std::atomic<int> refs{1};
@@ -92,8 +96,19 @@ struct CtxRef {
     void hold(ornith_hip_ctx *ctx) { c = ctx; c->refs++; }
     ~CtxRef() { if (c) ctx_drop(c); }
 };
-inline hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n) { return (hipError_t)c->pool.alloc(p, n); }
-inline hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b) { return (hipError_t)c->pool.get(n, b); }
+// The models' RoPE tables that no session uses, back to the device; the bytes
+size_t trim_tables(ornith_hip_ctx *c);
+// device memory, the kept tables and the pool's blocks given up for it if need be
+inline hipError_t dev_malloc(ornith_hip_ctx *c, void **p, size_t n) {
+    int e = c->pool.alloc(p, n);
+    if (e != hipSuccess && trim_tables(c) > 0) e = c->pool.alloc(p, n);
+    return (hipError_t)e;
+}
+inline hipError_t dev_get(ornith_hip_ctx *c, size_t n, DevBlock *b) {
+    int e = c->pool.get(n, b);
+    if (e != hipSuccess && trim_tables(c) > 0) e = c->pool.get(n, b);
+    return (hipError_t)e;
+}
 inline void dev_put(ornith_hip_ctx *c, const DevBlock &b) { c->pool.put(b); }
 
 // ---- tensors in the plane layout (oh_types.h) ---------------------------------------
@@ -150,6 +165,15 @@ struct OhLayer {
     ornith_hip_tensor *ffn_gate = nullptr, *ffn_up = nullptr, *ffn_down = nullptr;
 };
 
+// RoPE (cos, sin) per (position < cap, pair), shared by sessions of a model: it
+// goes with the last of them, or with the model that keeps it for the next
+struct RopeTable {
+    float2 *d = nullptr;
+    int cap = 0;
+    size_t bytes = 0;
+    ~RopeTable() { if (d) (void)hipFree(d); }
+};
+
 struct ornith_hip_model {
     ornith_hip_ctx *ctx = nullptr;
     CtxRef ref;
@@ -160,12 +184,9 @@ struct ornith_hip_model {
     bool any_full = false;        // a full-attention (GQA) layer exists
     ornith_hip_tensor *embd = nullptr, *out_norm = nullptr, *lm_head = nullptr;
     uint64_t bytes = 0;
-    // RoPE (cos, sin) of positions < rope_cap, shared by the model's sessions;
-    // the tables it outgrew stay until the model is freed
+    // the longest RoPE table so far, for the model's next sessions (rope_mu)
     std::mutex rope_mu;
-    float2 *rope = nullptr;
-    int rope_cap = 0;
-    std::vector<float2 *> rope_all;
+    std::shared_ptr<const RopeTable> rope;
 };
 
 // metadata view shared by the GGUF and synthetic paths
@@ -195,6 +216,7 @@ struct ornith_hip_session {
     int cap = 0, pos = 0, kvcap = 0;
     bool have_logits = false;
     std::vector<void *> allocs;   // the session's buffers, parts of its blocks (and the RoPE table)
+    std::shared_ptr<const RopeTable> rope_table;
     std::vector<size_t> asz;      // bytes requested for each of allocs
     std::vector<DevBlock> blocks; // device memory the session holds
     char *cur = nullptr;          // the last block's free part
@@ -422,6 +444,7 @@ ornith_hip_tensor *mt(const ornith_hip_model *m, const std::string &n);
 ornith_hip_tensor *mb(const ornith_hip_model *m, int l, const char *sfx);
 bool is_full(const ornith_hip_arch &a, int l);
 int infer_arch(ornith_hip_model *m, const Meta &md);
+void model_attach(ornith_hip_model *m, ornith_hip_ctx *c);   // a new model to its context
 int rec_begin(ornith_hip_session *s, hipStream_t st);
 int rec_end(ornith_hip_session *s, hipStream_t st, int kind, double bytes);
 bool keep(ornith_hip_session *s, int kind, double bytes);

@@ -111,10 +111,34 @@ int gguf_open(const char *path, Gguf &g) {
 
 } // namespace
 
+void model_attach(ornith_hip_model *m, ornith_hip_ctx *c) {
+    m->ctx = c;
+    m->ref.hold(c);
+    std::lock_guard<std::mutex> lk(c->models_mu);
+    c->models.push_back(m);
+}
+
+size_t trim_tables(ornith_hip_ctx *c) {
+    size_t bytes = 0;
+    std::lock_guard<std::mutex> lk(c->models_mu);
+    for (ornith_hip_model *m : c->models) {
+        std::lock_guard<std::mutex> lr(m->rope_mu);
+        if (m->rope && m->rope.use_count() == 1) {   // (sessions take it under the lock)
+            bytes += m->rope->bytes;
+            m->rope.reset();
+        }
+    }
+    return bytes;
+}
+
 extern "C" void ornith_hip_model_free(ornith_hip_model *m) {
     if (!m) return;
+    {
+        std::lock_guard<std::mutex> lk(m->ctx->models_mu);
+        auto &all = m->ctx->models;
+        all.erase(std::find(all.begin(), all.end(), m));
+    }
     for (auto *t : m->ts) ornith_hip_tensor_free(t);
-    for (float2 *r : m->rope_all) (void)hipFree(r);
     m->ctx->pool.trim(m);                         // its closed sessions' memory goes with the model
     delete m;
 }
@@ -270,8 +294,7 @@ extern "C" int ornith_hip_model_load(ornith_hip_ctx *ctx, const char *path, orni
     auto ie = g.kv.find("tokenizer.ggml.eos_token_id");
     if (ie != g.kv.end() && ie->second.len >= 4) memcpy(&md.eos, ie->second.val, 4);
     auto *m = new ornith_hip_model();
-    m->ctx = ctx;
-    m->ref.hold(ctx);
+    model_attach(m, ctx);
     for (auto &t : g.ts) {
         ornith_hip_tensor *dt;
         int st = ornith_hip_upload(ctx, t.name.c_str(), t.type, t.data, t.nbytes, t.nd, t.dims, &dt);

@@ -97,19 +97,34 @@ Act act_swiglu(const float *g, const float *u) {
 
 // RoPE cos/sin per (position, pair) with the reference's libm calls
 // (ot_rope_partial, src/ornith_tensor.c:167-178), once per model: a longer
-// session's table replaces it, half again as long at least
+// session's table takes the place of the model's, half again as long at least
+// where the device has the memory
 static int rope_table(ornith_hip_model *m, ornith_hip_session *s) {
     const ornith_hip_arch &a = m->a;
     const int half = a.hd / 2;
-    std::lock_guard<std::mutex> lk(m->rope_mu);
-    if (s->cap > m->rope_cap) {
+    int64_t cap = s->cap;
+    {
+        std::lock_guard<std::mutex> lk(m->rope_mu);
+        if (m->rope && m->rope->cap >= s->cap) s->rope_table = m->rope;
+        else if (m->rope) cap = std::max<int64_t>(cap, std::min<int64_t>((int64_t)m->rope->cap * 3 / 2, INT_MAX));
+    }
+    if (!s->rope_table) {
+        auto t = std::make_shared<RopeTable>();
+        auto bytes = [&]() { return (size_t)cap * half * sizeof(float2); };
+        hipError_t e = dev_malloc(m->ctx, (void **)&t->d, bytes() + 256);
+        if (e == hipErrorOutOfMemory && cap > s->cap) {
+            cap = s->cap;
+            e = dev_malloc(m->ctx, (void **)&t->d, bytes() + 256);
+        }
+        HCHK(e);
+        t->cap = (int)cap;
+        t->bytes = bytes();
         int rot = a.rope_dim;
         if (rot <= 0 || rot > a.hd) rot = a.hd;
-        const int cap = s->cap > m->rope_cap + m->rope_cap / 2 ? s->cap : m->rope_cap + m->rope_cap / 2;
         std::vector<float2> tab((size_t)cap * half);
         std::vector<float> freq((size_t)rot / 2);
         for (int i = 0; i < rot / 2; i++) freq[i] = powf(a.rope_theta, -2.0f * (float)i / (float)rot);
-        for (int p = 0; p < cap; p++)
+        for (int p = 0; p < (int)cap; p++)
             for (int i = 0; i < half; i++) {
                 float2 cs = {1.0f, 0.0f};
                 if (i < rot / 2) {
@@ -119,21 +134,14 @@ static int rope_table(ornith_hip_model *m, ornith_hip_session *s) {
                 }
                 tab[(size_t)p * half + i] = cs;
             }
-        float2 *d = nullptr;
-        HCHK(dev_malloc(m->ctx, (void **)&d, tab.size() * sizeof(float2) + 256));
-        const hipError_t e = hipMemcpy(d, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            (void)hipFree(d);
-            seterr("rope upload: %s", hipGetErrorString(e));
-            return ORNITH_HIP_ERR_DEVICE;
-        }
-        m->rope_all.push_back(d);
-        m->rope = d;
-        m->rope_cap = cap;
+        HCHK(hipMemcpy(t->d, tab.data(), t->bytes, hipMemcpyHostToDevice));
+        s->rope_table = t;
+        std::lock_guard<std::mutex> lk(m->rope_mu);
+        if (!m->rope || m->rope->cap < t->cap) m->rope = t;
     }
-    s->rope = m->rope;
+    s->rope = s->rope_table->d;
     s->allocs.push_back(s->rope);
-    s->asz.push_back((size_t)m->rope_cap * half * sizeof(float2));
+    s->asz.push_back(s->rope_table->bytes);
     return ORNITH_HIP_OK;
 }
 

@@ -36,8 +36,7 @@ extern "C" int ornith_hip_model_synth(ornith_hip_ctx *ctx, const ornith_hip_gen_
     float *tmp = nullptr;
     HCHK(dev_malloc(ctx, (void **)&tmp, mx * 4 + 256));
     auto *m = new ornith_hip_model();
-    m->ctx = ctx;
-    m->ref.hold(ctx);
+    model_attach(m, ctx);
     hipStream_t st = ctx->st;
     int status = ORNITH_HIP_OK;
     auto add_q = [&](const std::string &name, uint32_t type, int nd, uint64_t d0, uint64_t d1, uint64_t d2) {

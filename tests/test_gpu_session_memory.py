@@ -4,6 +4,8 @@ equal one, with other sessions open beside it, gives the bits that a session on
 fresh memory gives: prompt logits, greedy tokens and state. What the context
 keeps is one session's memory however many were opened in turn, and
 Context.trim gives it back."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -73,7 +75,7 @@ def test_closed_sessions_memory_serves_the_next():
     b.eval(p)
     a.free()
     b.free()
-    assert kept([4000]) == 2 * one
+    assert kept([4000]) == 2 * one - 4000 * 32 * 8   # the RoPE table is the model's
     x = clibs.gauss(8, "kept", 256 * 4096)
     ctx.quantize(clibs.Q4_K, x)
     enc = ctx.trim()
@@ -88,4 +90,47 @@ def test_closed_sessions_memory_serves_the_next():
     m.session(4000).free()
     m.free()
     assert ctx.trim() == 0
+    ctx.close()
+
+
+def test_rope_tables_go_with_their_sessions():
+    """A table that a longer session's outgrew goes with the last session that
+    reads it, the longest with Context.trim; a session that still reads one goes on."""
+    L = oa.lib()
+
+    def free_bytes():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert L.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    ctx = oa.Context(0)
+    m = ctx.synth(**clibs.C1)
+    p = np.random.default_rng(7).integers(0, clibs.C1["vocab"], 40).astype(np.int32)
+    first = m.session(60)
+    first.eval(p)
+    want, tokens = first.logits().copy(), first.generate(9)
+    first.free()
+    ctx.trim()
+    start = free_bytes()
+    table = 32 * 8                            # bytes of a position: pairs of a head of 64
+    short = m.session(400_000)
+    s = m.session(900_000)                    # a table of its own; short's was the model's
+    ctx.trim()
+    both = free_bytes()
+    short.eval(p)
+    assert np.array_equal(short.logits().view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(short.generate(9), tokens)
+    short.free()
+    ctx.trim()
+    # its KV cache, scores and table; half of the table's size of slack
+    least = 400_000 * (2 * 2 * (64 + 4) + 8 * 4 + table)
+    assert free_bytes() - both > least - 200_000 * table
+    s.free()
+    ctx.trim()
+    assert free_bytes() > start - (16 << 20)
+    s = m.session(60)
+    s.eval(p)
+    assert np.array_equal(s.logits().view(np.uint32), want.view(np.uint32))
+    s.free()
+    m.free()
     ctx.close()
