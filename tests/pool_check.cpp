@@ -34,7 +34,11 @@ void dev_release(void *p) {
     used -= it->second;
     live.erase(it);
 }
-size_t dev_unused(int) { return capacity - used; }
+int asked = 0;
+size_t dev_unused(int) {
+    asked++;
+    return capacity - used;
+}
 const DevMem kMem = {dev_alloc, dev_release, dev_unused};
 
 #define CHECK(x)                                                     \
@@ -129,6 +133,20 @@ int share() {
     return 0;
 }
 
+// blocks that come and go do not ask the device each time, and one that another
+// user filled is noticed all the same
+int asking() {
+    DevPool p(kMem, 0);
+    p.put(get(p, 100 * MiB));
+    asked = 0;
+    for (int i = 0; i < DevPool::kAsk - 1; i++) p.put(get(p, 100 * MiB));
+    CHECK(asked == 0 && used == 100 * MiB);
+    capacity = 1 * GiB;
+    p.put(get(p, 100 * MiB));
+    CHECK(asked == 1 && used == 0);
+    return 0;
+}
+
 // the end of one user leaves the blocks that served others
 int owners() {
     DevPool p(kMem, 0);
@@ -179,7 +197,7 @@ int other_pools() {
 
 const struct { const char *name; int (*run)(); } kChecks[] = {
     {"fit", fit}, {"unusable_bytes", unusable_bytes}, {"unusable_blocks", unusable_blocks},
-    {"bounds", bounds}, {"share", share}, {"owners", owners}, {"retry", retry}, {"other_pools", other_pools},
+    {"bounds", bounds}, {"share", share}, {"asking", asking}, {"owners", owners}, {"retry", retry}, {"other_pools", other_pools},
 };
 
 } // namespace
