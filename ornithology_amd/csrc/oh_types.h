@@ -321,9 +321,12 @@ typedef struct {
     int in, rows, xstride, ystride, adiv, cols;
 } oh_iq2rows;
 
-// Longest context of the decode step's exact walk for head dim hd: the
-// scores of the block's 256/hd heads stay in LDS, at most 48 KB of it
-// (8192 positions at hd 256, 6144 at 128, 3072 at 64).
+// Longest context of the decode step's exact walk for head dim hd (8192
+// positions at hd 256, 6144 at 128, 3072 at 64). The one-launch form
+// (exact_body) keeps the scores of a block's 256/hd heads in LDS, 48 KB at most;
+// the graph step's walk, which takes the same limit so that both give the same
+// bits, holds 16 positions a thread for the softmax (8192) and up to 148 KB of
+// LDS (its weights and four buffers of products).
 OH_HD static inline int exact_cap(int hd) {
     const int c = 12288 * hd / 256;
     return c < 8192 ? c : 8192;

@@ -1,6 +1,6 @@
 """The IQ2_XXS fallback rows turn a codebook entry into signed bytes with a
-table of byte masks (ornithology_amd/csrc/oh_mv.hip: iq2_sign_table,
-iq2_terms8): for the 7 stored sign bits s7 of a group, the eighth sign is
+table of byte masks (ornithology_amd/csrc/oh_iq2.h: iq2_sign_table; used in
+oh_mv.hip's iq2_terms and oh_kernels_iq2.hip): for the 7 stored sign bits s7 of a group, the eighth sign is
 their parity (the decoder's rule, src/ornith_quant.c:660-680), m byte j is
 0xff where sign j is negative, and (g ^ m) + (m & 0x01..) is the entry g with
 exactly those bytes negated, byte by byte without carries (every grid byte
