@@ -66,7 +66,7 @@ public:
             e = mem_.alloc(p, n);
         }
         std::lock_guard<std::mutex> lk(mu_);
-        most_ = 0;                            // there is less now
+        stale_ = true;                        // there is less now
         return e;
     }
     // a block of at least n bytes (contents undefined) from the pool or the device
@@ -94,7 +94,7 @@ public:
         bool ask;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            ask = bytes_ + b.n > most_ || ++puts_ >= kAsk;
+            ask = stale_ || bytes_ + b.n > most_ || ++puts_ >= kAsk;
         }
         const size_t unused = ask ? mem_.unused(device_) : 0;
         {
@@ -103,6 +103,7 @@ public:
                 const size_t share = (unused + bytes_ + b.n) / kShare;
                 most_ = share < kBytes ? share : kBytes;
                 puts_ = 0;
+                stale_ = false;
             }
             const bool keep = b.n <= most_;
             while ((keep && count_ == kBlocks) || (count_ > 0 && bytes_ + (keep ? b.n : 0) > most_)) old[n++] = take(0);
@@ -154,5 +155,6 @@ private:
     int count_ = 0;
     size_t bytes_ = 0;
     size_t most_ = 0;                     // what bytes_ may be, by the device's last answer
-    int puts_ = 0;                        // since then
+    bool stale_ = true;                   // it has to be asked again
+    int puts_ = 0;                        // blocks returned since
 };

@@ -6,7 +6,12 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <atomic>
 #include <map>
+#include <mutex>
+#include <set>
+#include <thread>
+#include <vector>
 
 namespace {
 
@@ -14,18 +19,19 @@ constexpr size_t MiB = (size_t)1 << 20, GiB = (size_t)1 << 30;
 size_t capacity = 288 * GiB, used = 0;
 uintptr_t next_addr = 0x1000;
 std::map<void *, size_t> live;
-int allocs = 0;
+std::mutex dev_mu;
 
 int dev_alloc(void **p, size_t n) {
+    std::lock_guard<std::mutex> lk(dev_mu);
     if (used + n > capacity) return 2;
     *p = (void *)next_addr;
     next_addr += n + 256;
     live[*p] = n;
     used += n;
-    allocs++;
     return 0;
 }
 void dev_release(void *p) {
+    std::lock_guard<std::mutex> lk(dev_mu);
     auto it = live.find(p);
     if (it == live.end()) {
         printf("a block that is not live was released\n");
@@ -36,6 +42,7 @@ void dev_release(void *p) {
 }
 int asked = 0;
 size_t dev_unused(int) {
+    std::lock_guard<std::mutex> lk(dev_mu);
     asked++;
     return capacity - used;
 }
@@ -147,6 +154,39 @@ int asking() {
     return 0;
 }
 
+// several threads: every block is in one place, none is lost, the bounds hold
+int threads() {
+    DevPool p(kMem, 0);
+    std::vector<std::thread> ts;
+    std::atomic<int> bad{0};
+    std::mutex mu;
+    std::set<void *> out;
+    for (int t = 0; t < 8; t++)
+        ts.emplace_back([&, t]() {
+            unsigned r = 17u * (unsigned)t + 1;
+            for (int i = 0; i < 2000; i++) {
+                r = r * 1664525u + 1013904223u;
+                DevBlock b;
+                if (p.get((1 + (r >> 8) % 200) * MiB, &b) != 0) bad++;
+                {
+                    std::lock_guard<std::mutex> lk(mu);
+                    if (!out.insert(b.p).second) bad++;
+                }
+                {
+                    std::lock_guard<std::mutex> lk(mu);
+                    out.erase(b.p);
+                }
+                p.put(b);
+                if (r % 97 == 0) p.trim();
+            }
+        });
+    for (std::thread &t : ts) t.join();
+    CHECK(bad == 0 && used <= DevPool::kBytes && (int)live.size() <= DevPool::kBlocks);
+    p.trim();
+    CHECK(used == 0 && live.empty());
+    return 0;
+}
+
 // the end of one user leaves the blocks that served others
 int owners() {
     DevPool p(kMem, 0);
@@ -197,7 +237,7 @@ int other_pools() {
 
 const struct { const char *name; int (*run)(); } kChecks[] = {
     {"fit", fit}, {"unusable_bytes", unusable_bytes}, {"unusable_blocks", unusable_blocks},
-    {"bounds", bounds}, {"share", share}, {"asking", asking}, {"owners", owners}, {"retry", retry}, {"other_pools", other_pools},
+    {"bounds", bounds}, {"share", share}, {"asking", asking}, {"owners", owners}, {"threads", threads}, {"retry", retry}, {"other_pools", other_pools},
 };
 
 } // namespace

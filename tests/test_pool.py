@@ -8,7 +8,7 @@ import pytest
 
 import clibs
 
-CHECKS = ("fit", "unusable_bytes", "unusable_blocks", "bounds", "share", "asking", "owners", "retry", "other_pools")
+CHECKS = ("fit", "unusable_bytes", "unusable_blocks", "bounds", "share", "asking", "owners", "threads", "retry", "other_pools")
 
 
 @pytest.fixture(scope="module")
